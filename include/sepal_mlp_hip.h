@@ -88,8 +88,8 @@ SEPAL_HIP_API int32_t sepal_hip_quantize_gate_up_s8(const void* gate, const void
  * 16-bit X rows of whole 16-byte chunks and store STORE / ADD outputs in 16-column tiles; other strides and the last
  * N mod 16 columns are staged in the workspace (a contiguous copy of X; one zero-padded 16-row weight tile whose
  * float32 outputs are stored or added into Y). `config` -1 picks a path by T and N (at
- * T <= 16 with a 16-bit X the M <= 16 stack's pass kernels where the shape fits them; small-M streaming at T <= 32 with
- * N < 8192; on the large-M path grids too small to fill the chip may split K over blocks; a row's bits then depend on
+ * T <= 16 with a 16-bit X the M <= 16 stack's pass kernels where the shape fits them; at T <= 64 with a 16-bit X a
+ * kernel that splits K over waves and blocks, at 49 to 64 rows for N <= 48 x CUs only; on the large-M path grids too small to fill the chip may split K over blocks; a row's bits then depend on
  * T); 0 forces the large-M
  * tiled path without a split of K (a row's bits do not depend on the batch, as the reference's), 1 the small-M
  * weight-streaming path, 2 the small-M path without a split of K (the whole K of a column block in one block; K at
@@ -120,10 +120,10 @@ SEPAL_HIP_API int32_t sepal_hip_quantize_rows_s8(const void* x, int32_t x_type, 
  * large-M path reproduces cpu-q8 bit for bit. act_block = K (one scale per token): y = (f_0 * ws_0, then
  * fma(f_b, ws_b, y)) * xs. Epilogues STORE / ADD / SWIGLU (silu with the cpu-q8 exp polynomial); Y float32
  * [T, ld_y], or y_type for SWIGLU. K a multiple of 128; strides multiples of 16; 16-byte aligned pointers. `config`
- * -1 takes the small-M path up to 64 rows (above 32 rows only for N < 8192; at T <= 16 with a float32 Y the M <= 16
- * stack's q8 passes where the shape fits them), 0 the large-M path, 1 the small-M path,
- * 2 the small-M path with the chain whole; the small-M path splits K across blocks when N is narrow, which keeps the
- * sums exact but adds the splits' partial chains (within tolerance, not bit for bit); config 2 keeps the chain whole
+ * -1 takes a small-M path up to 64 rows (at T <= 16 with a float32 Y the M <= 16 stack's q8 passes where the shape
+ * fits them, else a kernel that splits K over waves and blocks), 0 the large-M path, 1 the streaming small-M path,
+ * 2 the streaming path with the chain whole; the small-M paths split K, which keeps the int32 group sums exact but adds
+ * the splits' partial chains (within tolerance, not bit for bit); config 2 keeps the chain whole
  * (bit for bit).
  * Replaces kernel_i8_z + finish_tile (runner/src/cpu/gemm_kernels_avx512.cpp:67-115, gemm.cpp:417-447, 545-569)
  * with per-group scales (the per-channel launch_gemm_s8 is sepal_hip_gemm_s8). */

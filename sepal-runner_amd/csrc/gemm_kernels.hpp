@@ -8,8 +8,8 @@ namespace sepal::hip {
 // Rows at or below which the multiplies take the weight-streaming small-M path.
 inline constexpr std::size_t kSmallM = 64;
 
-// Default routing of the q8 multiply (config -1): the small-M (streaming) kernels up to kSmallM rows, except above 32
-// rows with N >= 8192, where the large-M kernels are faster (gate/up 19456 x 2560 at T = 40-64: 28-30 against 41-43 us
+// Default routing of the q8 multiply (config -1) for what mid_gemm_plan refuses (offsets beyond 32 bits): the small-M
+// (streaming) kernels up to kSmallM rows, except above 32 rows with N >= 8192, where the large-M kernels are faster (gate/up 19456 x 2560 at T = 40-64: 28-30 against 41-43 us
 // per token, 35-37 against 43-44 per 128; 12288 x 2560: 29-33 against 35) and also bit-exact to cpu-q8.
 inline bool q8_streams(std::size_t t, std::size_t n) { return t <= kSmallM && (t <= 32 || n < 8192); }
 
@@ -152,6 +152,17 @@ bool small_q8_group_sums(const GemmArgs& a, hipStream_t stream);
 // ... and for the Store / Add multiply (float32 Y through K-parts and the parts sum).
 bool small_gemm_plan_q8_parts(const GemmArgs& a, SmallGemmPlan& plan);
 void launch_small_gemm_q8_parts(const GemmArgs& a, const SmallGemmPlan& plan, hipStream_t stream);
+// y [t, n] (any row stride) = or += (add) the in-order sum of `parts` float32 planes part [parts][t][n].
+void launch_parts_add(int parts, bool add, std::size_t t, std::size_t n, const float* part, float* y, std::size_t ld_y,
+                      hipStream_t stream);
+// One multiply of up to 64 rows (mid.hip; config -1): w8g with a 16-bit X, or q8. mid_gemm_plan returns false for what
+// the kernel does not take (another T, config or X type, offsets beyond 32 bits).
+struct MidGemmPlan {
+    int nt;     // 16-row weight tiles per block
+    int parts;  // K-parts (1 for SwiGLU)
+};
+bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan);
+void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStream_t stream);
 // x bf16 [t, hidden] -> h binary16 [t, inter] -> part float32 [parts][t][hidden] -> y float32 [t, hidden] and, when
 // xn is set, xn bf16 [t, hidden] = RMSNorm(y) (cpu-q8 order, identity weight). stream_w: w_gu and w_d in the stream
 // layout (launch_stream_layout; the same bits).

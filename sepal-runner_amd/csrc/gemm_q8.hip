@@ -1115,6 +1115,11 @@ void dispatch_path(const GemmArgs& a, hipStream_t stream) {
             return;
         }
     }
+    MidGemmPlan mid;  // up to 64 rows by default: K split over waves and blocks
+    if (mid_gemm_plan(a, true, mid)) {
+        launch_mid_gemm(a, true, mid, stream);
+        return;
+    }
     const bool small = a.config == 1 || (a.config < 0 && q8_streams(a.t, a.n));
     if (small) launch_stream_q8(a, stream);
     else launch_big<EP, YT, PT, MODE_CHAIN>(a, stream);

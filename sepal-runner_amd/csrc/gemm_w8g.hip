@@ -1433,7 +1433,8 @@ void launch_big(const GemmArgs& a, hipStream_t stream) {
 }
 
 // Whether a problem takes the small-M (weight-streaming) kernels: they write float32 (or SwiGLU outputs); a binary16
-// Store always takes the large-M kernels. By default they take T <= 32 with N < 8192: measured on the model's weight
+// Store always takes the large-M kernels. By default they take T <= 32 with N < 8192 of what the kernels asked first
+// (dispatch_path) refuse, and of the two multiplies of a float32 X: measured on the model's weight
 // shapes, the large-M kernels' small-grid plan (64-row blocks, K split) is faster above 32 rows (the streaming kernels
 // double their time from 33 rows, at 64-row tiles) and at any T for N >= 8192 (gate/up 19456 x 2560: 20 against
 // 24 us at T = 1), and the streaming kernels are faster for the narrow, long-K down shape (2560 x 9728: 22.5 against
@@ -1455,6 +1456,11 @@ void dispatch_path(const GemmArgs& a, hipStream_t stream) {
         SmallGemmPlan plan;
         if (a.config < 0 && a.t <= 16 && small_gemm_plan(a, plan)) {
             launch_small_gemm_w8g(a, plan, stream);
+            return;
+        }
+        MidGemmPlan mid;  // up to 64 rows by default: K split over waves and blocks
+        if (mid_gemm_plan(a, false, mid)) {
+            launch_mid_gemm(a, false, mid, stream);
             return;
         }
     }

@@ -994,6 +994,12 @@ void launch_pass_w(const GemmArgs& a, const stack::PassParams& p, std::size_t ld
 
 } // namespace
 
+void launch_parts_add(int parts, bool add, std::size_t t, std::size_t n, const float* part, float* y, std::size_t ld_y,
+                      hipStream_t stream) {
+    launch_parts_sum(parts, add, t, n, part, y, ld_y, stream);
+    check_launch("parts sum launch");
+}
+
 bool small_gemm_plan(const GemmArgs& a, SmallGemmPlan& plan) {
     constexpr std::size_t kLds = 160u << 10;
     constexpr int kMaxPairs = stack::kWorkers * stack::kPairs;

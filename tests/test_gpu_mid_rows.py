@@ -1,0 +1,109 @@
+"""The multiplies of up to 64 rows that split K over waves and blocks (MI355X only): w8g with bf16 / binary16 X and q8 in
+both activation-scale modes, at the edges of the kernel's row tiles (16, 32, 48, 64), of its blocks of 2, 3 or 5 weight
+tiles (a last block with tiles missing), of its K-parts and of its waves (fewer groups than waves), with padded strides.
+
+Reference: float64 of the dequantized operands. Bound: a float32 sum of K products and G group links is within
+(K + G + 8) 2^-24 sum |x_k w_k| of it (each product and addition rounds once; the q8 sums of a group are exact); SwiGLU
+adds |d silu(g) u| <= 1.1 |u| dg + |silu(g)| du and a few ulp of its own."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def sm():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import sepal_mlp
+    sepal_mlp.library()
+    return sepal_mlp
+
+
+def _swiglu(z):
+    t, n = z.shape
+    z = z.view(t, n // 128, 2, 64)
+    gate, up = z[:, :, 0, :], z[:, :, 1, :]
+    return (gate.reshape(t, n // 2), up.reshape(t, n // 2))
+
+
+def _check(y, ref, mag, u):
+    """|y - ref| within u * mag of the sums, elementwise."""
+    assert torch.isfinite(y).all()
+    excess = (y.double() - ref).abs() - u * mag
+    assert (excess <= 0).all(), excess.max().item()
+
+
+def _check_swiglu(h, z, mag, u, type_eps):
+    g, up = _swiglu(z)
+    dg, du = _swiglu(u * mag)
+    silu = g / (1 + torch.exp(-g))
+    ref = silu * up
+    bound = 1.1 * up.abs() * dg + silu.abs() * du + dg * du + 2.0**-20 * ref.abs() + type_eps * ref.abs() + 1e-7
+    assert ((h.double() - ref).abs() <= bound).all()
+
+
+SHAPES = [
+    # t, n, k: one tile and one group; tiles short of a block; groups short of the waves; K-parts; a wide grid; NT 2 / 3 / 5
+    (17, 16, 128), (20, 144, 128), (31, 48, 640), (32, 2560, 9728), (33, 80, 1152), (48, 1008, 512), (49, 128, 384),
+    (63, 12288, 256), (64, 2576, 1280), (40, 20608, 256), (64, 256, 9728), (5, 640, 384), (16, 2048, 3200),
+]
+
+
+@pytest.mark.parametrize("t,n,k", SHAPES)
+def test_up_to_64_rows(sm, t, n, k):
+    print("[case] mid rows", t, n, k, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1000 * t + n + k)
+    w = (torch.randn(n, k, generator=g, device="cuda") * 0.02).half()
+    x = torch.randn(t, k + 16, generator=g, device="cuda")[:, :k]
+    u = (k + k // 128 + 8) * 2.0**-24
+    q, s = sm.quantize_group_s8(w)
+    wpad = torch.zeros(n, k + 32, dtype=torch.int8, device="cuda")
+    wpad[:, :k] = q
+    deq = (q.double().view(n, k // 128, 128) * s.double()[:, :, None]).view(n, k)
+    for dt in (torch.bfloat16, torch.float16):
+        xp = torch.zeros(t, k + 16, dtype=dt, device="cuda")
+        xp[:, :k] = x.to(dt)
+        xb = xp[:, :k]
+        ref, mag = xb.double() @ deq.T, xb.double().abs() @ deq.abs().T
+        y = torch.full((t, n + 4), 7.0, device="cuda")
+        sm.gemm_w8g(xb, wpad[:, :k], s, y=y[:, :n])
+        _check(y[:, :n], ref, mag, u)
+        assert (y[:, n:] == 7.0).all()
+        y0 = torch.randn(t, n, generator=g, device="cuda")
+        ya = sm.gemm_w8g(xb, q, s, y=y0.clone(), epilogue=sm.ADD)
+        _check(ya, ref + y0.double(), mag + y0.double().abs() + ref.abs(), u)
+        if n % 128 == 0:
+            for yt, eps in ((torch.float32, 0.0), (torch.float16, 2.0**-11), (torch.bfloat16, 2.0**-8)):
+                _check_swiglu(sm.gemm_w8g(xb, q, s, epilogue=sm.SWIGLU, y_dtype=yt), ref, mag, u, eps)
+    for block in (k, 128):
+        xq, xs = sm.quantize_rows_s8(x.contiguous(), block=block)
+        xd = (xq.double().view(t, k // block, block) * xs.double()[:, :, None]).view(t, k)
+        ref, mag = xd @ deq.T, xd.abs() @ deq.abs().T
+        _check(sm.gemm_q8(xq, xs, q, s, act_block=block), ref, mag, u)
+        if n % 128 == 0:
+            _check_swiglu(sm.gemm_q8(xq, xs, q, s, act_block=block, epilogue=sm.SWIGLU), ref, mag, u, 0.0)
+        if n % 256 == 0:
+            hq, hs = sm.gemm_q8_swiglu_quantize(xq, xs, q, s, act_block=block)
+            h = sm.gemm_q8(xq, xs, q, s, act_block=block, epilogue=sm.SWIGLU)
+            rq, rs = sm.quantize_rows_s8(h, block=128)
+            assert torch.equal(hq, rq) and torch.equal(hs, rs)
+
+
+@pytest.mark.parametrize("t", [17, 48, 64])
+def test_rows_do_not_see_each_other(sm, t):
+    """A row's bits depend on that row alone at one T; a row of infinities stays in its row; the second call repeats the
+    first one's bits (the K-parts and waves are added in a fixed order)."""
+    n, k = 2560, 2560
+    g = torch.Generator(device="cuda").manual_seed(t)
+    q, s = sm.quantize_group_s8((torch.randn(n, k, generator=g, device="cuda") * 0.02).half())
+    x = torch.randn(t, k, generator=g, device="cuda").bfloat16()
+    a = sm.gemm_w8g(x, q, s)
+    assert torch.equal(a, sm.gemm_w8g(x, q, s))
+    x2 = torch.randn(t, k, generator=g, device="cuda").bfloat16()
+    x2[t // 2] = x[t // 2]
+    x2[0] = float("inf")
+    b = sm.gemm_w8g(x2, q, s)
+    assert torch.equal(a[t // 2], b[t // 2])
+    assert torch.isfinite(b[1:]).all() and not torch.isfinite(b[0]).any()
