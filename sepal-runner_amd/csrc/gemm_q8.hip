@@ -8,7 +8,8 @@
 //   epilogue: Store, Add (y + acc), SwiGLU (silu with the cpu-q8 exp polynomial; gate/up rows in the 64-row interleave)
 // Every step is one IEEE operation in the reference's order, so the large-M path equals cpu-q8 bit for bit.
 //
-// Large-M path: 128 x 256 tiles of 8 waves, each 64 x 64 outputs (2 x 2 blocks of MFMA 32x32x32 i8); K in steps of
+// Large-M path: 128 x 256 tiles (or smaller ones, gemm_chain) of 8 waves, each 64 x 64 outputs (2 x 2 blocks of MFMA
+// 32x32x32 i8); K in steps of
 // one group (128 bytes) through three LDS stages, filled straight from global memory (global_load_lds, whole 128-byte
 // rows per 8 lanes) two groups ahead; the int32 sums of a group are turned into the float chain in registers before
 // the next group starts (a second set of accumulators holds the chain).
@@ -114,33 +115,36 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef const __attribute__((address_space(1))) void global_void;
 
-// The chain modes' epilogue of a 128 x 256 tile: acc[i][q][r] holds the chain of output (row m0 + wm 64 + 32 i +
-// 8 (r / 4) + 4 (lane / 32) + r % 4, column col[q]); per token it is multiplied by the row's activation scale here.
-// hb: LDS scratch of 32 KB (kSwigluQ8 only; free when called).
+// The chain modes' epilogue of a tile of WM x WN waves, each 32 MBLK rows x 64 columns: acc[i][q][r] holds the chain of
+// output (row m0 + 32 MBLK wm + 32 i + 8 (r / 4) + 4 (lane / 32) + r % 4, column col[q]); per token it is multiplied by
+// the row's activation scale here. hb: LDS scratch of 256 bytes per tile row (kSwigluQ8 only; free when called).
 // FAST_SILU: the SwiGLU of the per-token chain (swiglu_q8<true>); the per-128 chain and the AVX2 int8 multiply's
 // whole-K form keep the cpu-q8 silu.
-template <int EP, int YT, bool PER_TOKEN, bool FAST_SILU = PER_TOKEN>
-__device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][2][16], int m0, int n0, int wm, int ib, int hh,
+template <int EP, int YT, bool PER_TOKEN, int WM, int WN, int MBLK, bool FAST_SILU = PER_TOKEN>
+__device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[MBLK][2][16], int m0, int n0, int wm, int ib, int hh,
                                                int lane, int tid, const int (&col)[2], float* hb) {
-    constexpr int BM = 128;
+    constexpr int WR = 32 * MBLK, BM = WR * WM, BN = 64 * WN;
     if constexpr (EP == kSwigluQ8) {
         // The tile's 128 output columns are one quantization block. H goes through LDS (the first W stage, free after
-        // the loop) in two halves of 64 columns: 128 rows of 256 bytes, 16-byte chunk c of row r at c ^ (r % 16). Thread
-        // (row, q) takes 16 columns of one row from each half: the max over them, the four quarters combined through
-        // LDS, the scale, and 32 int8 values stored as two 16-byte chunks. max is exact in any order, so this equals
+        // the loop) in two halves of 64 columns: rows of 256 bytes, 16-byte chunk c of row r at c ^ (r % 16). Thread
+        // (row, part) takes VC = 64 / PARTS columns of one row from each half: the max over them, the parts combined
+        // through LDS, the scale, and the int8 values stored as two runs. max is exact in any order, so this equals
         // quantize_rows on the float32 H (rule RECIPROCAL).
-        __shared__ float lds_amax[4][BM];
+        static_assert(BN == 256, "a tile's outputs are one block of 128 columns");
+        constexpr int PARTS = 64 * WM * WN / BM, VC = 64 / PARTS;
+        static_assert(VC == 8 || VC == 16, "whole 8- or 16-byte stores");
+        __shared__ float lds_amax[PARTS][BM];
         const int c = 32 * hh + lane % 32;  // this lane's column within its half (half ib)
         const int row_l = tid % BM, quarter = tid / BM;
-        float hv[32];
+        float hv[2 * VC];
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             if (ib == half) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < MBLK; ++i)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const int rl = wm * 64 + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
+                        const int rl = wm * WR + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
                         float v0 = acc[i][0][r], v1 = acc[i][1][r];
                         if constexpr (PER_TOKEN) {
                             const float xs = p.xs[static_cast<std::size_t>(min(m0 + rl, p.t - 1)) * p.ld_xs];
@@ -152,18 +156,18 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][
             }
             __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const float4 v = *reinterpret_cast<const float4*>(hb + row_l * 64 + (((4 * quarter + j) ^ (row_l % 16)) * 4));
-                hv[16 * half + 4 * j] = v.x;
-                hv[16 * half + 4 * j + 1] = v.y;
-                hv[16 * half + 4 * j + 2] = v.z;
-                hv[16 * half + 4 * j + 3] = v.w;
+            for (int j = 0; j < VC / 4; ++j) {
+                const float4 v = *reinterpret_cast<const float4*>(hb + row_l * 64 + (((VC / 4 * quarter + j) ^ (row_l % 16)) * 4));
+                hv[VC * half + 4 * j] = v.x;
+                hv[VC * half + 4 * j + 1] = v.y;
+                hv[VC * half + 4 * j + 2] = v.z;
+                hv[VC * half + 4 * j + 3] = v.w;
             }
             __syncthreads();
         }
         float m = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 32; ++j) {
+        for (int j = 0; j < 2 * VC; ++j) {
             const float a = fabsf(hv[j]);
             m = a > m ? a : m;
         }
@@ -171,14 +175,14 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][
         __syncthreads();
         m = lds_amax[0][row_l];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) m = lds_amax[w][row_l] > m ? lds_amax[w][row_l] : m;
+        for (int w = 1; w < PARTS; ++w) m = lds_amax[w][row_l] > m ? lds_amax[w][row_l] : m;
         const float scale = m > 0.0f ? __fdiv_rn(m, 127.0f) : 1.0f;
         const float inverse = __fdiv_rn(1.0f, scale);
         const int row = m0 + row_l;
         if (row < p.t) {
-            unsigned packed[8];
+            unsigned packed[VC / 2];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < VC / 2; ++j) {
                 packed[j] = 0u;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -187,9 +191,14 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][
                     packed[j] |= (static_cast<unsigned>(static_cast<int>(qv)) & 0xFFu) << (8 * e);
                 }
             }
-            signed char* dst = static_cast<signed char*>(p.y) + static_cast<std::size_t>(row) * p.ld_y + n0 / 2 + 16 * quarter;
-            *reinterpret_cast<u32x4*>(dst) = u32x4{packed[0], packed[1], packed[2], packed[3]};
-            *reinterpret_cast<u32x4*>(dst + 64) = u32x4{packed[4], packed[5], packed[6], packed[7]};
+            signed char* dst = static_cast<signed char*>(p.y) + static_cast<std::size_t>(row) * p.ld_y + n0 / 2 + VC * quarter;
+            if constexpr (VC == 16) {
+                *reinterpret_cast<u32x4*>(dst) = u32x4{packed[0], packed[1], packed[2], packed[3]};
+                *reinterpret_cast<u32x4*>(dst + 64) = u32x4{packed[4], packed[5], packed[6], packed[7]};
+            } else {
+                *reinterpret_cast<uint2*>(dst) = make_uint2(packed[0], packed[1]);
+                *reinterpret_cast<uint2*>(dst + 64) = make_uint2(packed[2], packed[3]);
+            }
             if (quarter == 0) p.ys[static_cast<std::size_t>(row) * p.ld_ys + n0 / 256] = scale;
         }
         return;
@@ -197,7 +206,7 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][
     // A whole tile needs no bounds checks: the row and the wave's column base are wave-uniform (scalar registers) and
     // the lane adds a 32-bit offset, so a store (and, per token, the row scale's load) costs no vector address
     // arithmetic.
-    if (m0 + BM <= p.t && n0 + 256 <= p.n) {
+    if (m0 + BM <= p.t && n0 + BN <= p.n) {
         constexpr unsigned ES = YT == SEPAL_HIP_F32 ? 4 : 2;
         const int wmu = __builtin_amdgcn_readfirstlane(wm), ibu = __builtin_amdgcn_readfirstlane(ib),
                   hhu = __builtin_amdgcn_readfirstlane(hh);
@@ -206,10 +215,10 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][
         const unsigned xoff = lrow * static_cast<unsigned>(p.ld_xs) * 4u;
         char* const yb = static_cast<char*>(p.y);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < MBLK; ++i) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const std::size_t row = static_cast<std::size_t>(m0 + wmu * 64 + i * 32 + 8 * (r / 4) + (r % 4));
+                const std::size_t row = static_cast<std::size_t>(m0 + wmu * WR + i * 32 + 8 * (r / 4) + (r % 4));
                 float v0 = acc[i][0][r], v1 = acc[i][1][r];
                 if constexpr (PER_TOKEN) {
                     const float xs = *reinterpret_cast<const float*>(
@@ -232,10 +241,10 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[2][
         return;
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < MBLK; ++i) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int row = m0 + wm * 64 + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
+            const int row = m0 + wm * WR + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
             if (row >= p.t) continue;
             float v0 = acc[i][0][r], v1 = acc[i][1][r];
             if constexpr (PER_TOKEN) {
@@ -506,7 +515,7 @@ __global__ void __launch_bounds__(512) gemm_big(const Params p) {
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = __fmul_rn(static_cast<float>(tot[i][j][r]), wsrow[j][0]);
     }
 
-    chain_epilogue<EP, YT, PER_TOKEN, PER_TOKEN && MODE == MODE_CHAIN>(p, acc, m0, n0, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
+    chain_epilogue<EP, YT, PER_TOKEN, 2, 4, 2, PER_TOKEN && MODE == MODE_CHAIN>(p, acc, m0, n0, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
 }
 
 // ---- the chain, two wave groups in alternation (gemm_chain) ---------------------------------------------------------
@@ -533,17 +542,32 @@ __global__ void __launch_bounds__(512) gemm_big(const Params p) {
 // previous L slot), so both shares are complete by the barrier that ends slot 2g + 1, before group g + 1 is first
 // read; every wave issues, reads and waits alike (only B's extra barrier at the start and A's at the end differ), so
 // the kernel has no branch between the groups' code. The launcher uses this kernel when every offset fits 32 bits.
+//
+// Smaller tiles (WM x WN waves of 32 MBLK rows x 64 columns; chain_plan below picks) fill the chip where the 128 x 256
+// grid cannot. Eight waves alternate as above; blocks of 2, 4 or 6 waves run L(g), a barrier, M(g) and go straight on to
+// L(g + 1). At 2560 x 9728 (76 groups) a group takes 1.05 us on 128 x 256 tiles, 0.68 on 128 x 128, 0.61 on 96 x 128, 0.49 on
+// 64 x 128 and 0.41 on 32 x 128. Bound of the small ones (ablations, 64 x 128, 52 us at T = 640 with the fragments read a
+// group ahead): 29 us without the links, 32 without the loads, 52 without the MFMAs or the fragment reads: a wave's VALU
+// instructions and its loads' issue run in turn. Four to six stages (36 to 45 us where three take 37 to 46) and
+// fragments read one group ahead (47 to 52) gave nothing.
 struct ChainParams {
     Params p;
+    int total;  // tiles of this launch
+    int id0;    // (tiles below 128 x 256) -1: the grid p.tiles_m x p.tiles_n of the kernel's own tiles; else the kernel's tiles inside the 128 x 256
+                // tiles id0, id0 + 1, ... of the grid p.tiles_m x p.tiles_n of those
     unsigned x_bytes, w_bytes, ws_bytes, xs_bytes;  // extents of X, W and their scales (buffer ranges)
 };
 
-template <int EP, int YT, bool PER_TOKEN>
-__global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
+template <int EP, int YT, bool PER_TOKEN, int WM, int WN, int MBLK>
+__global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM * WN == 2 ? 1 : 2))) gemm_chain(const ChainParams cp) {
     const Params& p = cp.p;
-    constexpr int BM = 128, BN = 256;
-    // a wave's loads per group: its operand shares, its 2 weight scales and, per 128, one activation scale
-    constexpr int XDMA = BM / 64, WDMA = BN / 64, NLD = XDMA + WDMA + 2 + (PER_TOKEN ? 0 : 1);
+    constexpr int NW = WM * WN, WR = 32 * MBLK, BM = WR * WM, BN = 64 * WN, NB = 2 * MBLK;
+    constexpr bool PP = NW == 8;  // two wave groups in alternation
+    constexpr int RW = BM / NW;   // per 128: tile rows whose activation scale a wave loads
+    // a wave's loads per group: its operand shares (1 KB each; with 6 waves the last of the weights' turn repeats), its
+    // 2 weight scales and, per 128, one activation scale
+    constexpr int XDMA = BM / 8 / NW, WDMA = (BN / 8 + NW - 1) / NW, NLD = XDMA + WDMA + 2 + (PER_TOKEN ? 0 : 1);
+    static_assert(XDMA * NW * 8 == BM && RW * NW == BM && RW <= 64, "whole shares");
     __shared__ __align__(1024) u32x4 lx0[BM * 8], lx1[BM * 8], lx2[BM * 8];
     __shared__ __align__(1024) u32x4 lw0[BN * 8], lw1[BN * 8], lw2[BN * 8];
     // per 128: the tile rows' activation scales of group g in ring slot (xb + g) mod 4. Four slots, not three: group
@@ -567,12 +591,12 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
 
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);  // wave-uniform: LDS destinations stay scalar
-    const bool group_b = wave >= 4;
-    const int wm = wave % 2, wn = wave / 2;
+    const bool group_b = PP && wave >= 4;
+    const int wm = wave % WM, wn = wave / WM;
     // persistent: one block per CU; block b works through the contiguous range [lo, hi) of logical tiles of its XCD
     // (b mod 8), every (gridDim.x / 8)-th from lo + b / 8, so the XCD's blocks run consecutive tiles at a time (they
     // share its L2)
-    const int total = p.tiles_m * p.tiles_n;
+    const int total = cp.total;
     int cur, hi, stride;
     {
         const int nx = static_cast<int>(gridDim.x) / 8, xcd = static_cast<int>(blockIdx.x) % 8;
@@ -589,34 +613,50 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
     const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(const_cast<signed char*>(p.w), 0, static_cast<int>(cp.w_bytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t wsres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.ws), 0, static_cast<int>(cp.ws_bytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t xsres = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.xs), 0, static_cast<int>(cp.xs_bytes), 0x00020000);
-    // a wave's share of a group's loads: direct load e fills LDS kilobyte wave + 8 e = rows 8 wave + 64 e + {0..7};
-    // lane l writes slot l % 8 of row 8 wave + 64 e + l / 8, which holds chunk (l % 8) ^ sw8(row) = (l % 8) ^
-    // ((4 wave + l / 16) & 7); rows past T or N repeat the last row (never stored)
+    // a wave's share of a group's loads: direct load e fills LDS kilobyte kb = wave + NW e = rows 8 kb + {0..7}; lane l
+    // writes slot l % 8 of row 8 kb + l / 8, which holds chunk (l % 8) ^ sw8(row) = (l % 8) ^ ((4 kb + l / 16) & 7): NW is
+    // even, so every e has the same chunk; rows past T or N repeat the last row (never stored)
+    static_assert(NW % 2 == 0, "one chunk per lane for all of a wave's loads");
     const int chunk = (lane % 8) ^ ((4 * wave + lane / 16) & 7);
+    const auto wkb = [&](int e) __attribute__((always_inline)) {
+        if constexpr (BN / 8 % NW == 0) return wave + NW * e;
+        else return min(wave + NW * e, BN / 8 - 1 - ((BN / 8 - 1 - wave) & 1));  // (the last of the wave's parity)
+    };
     const int ib = wn / 2, hh = wn % 2;
     const int colrel[2] = {128 * ib + 32 * hh + lane % 32, 128 * ib + 64 + 32 * hh + lane % 32};
     // the tile's origin and the offsets that depend on it
     int m0, n0, xoff[XDMA], woff[WDMA], ws_off0, ws_off1, xs_off;
     const auto set_tile = [&]() __attribute__((always_inline)) {
         int tm, tn;
-        tile_from_id(cur, p.tiles_m, p.tiles_n, tm, tn);
-        m0 = tm * BM;
-        n0 = tn * BN;
+        if constexpr (BM == 128 && BN == 256) {
+            tile_from_id(cur, p.tiles_m, p.tiles_n, tm, tn);
+            m0 = tm * BM;
+            n0 = tn * BN;
+        } else if (cp.id0 < 0) {
+            tile_from_id(cur, p.tiles_m, p.tiles_n, tm, tn);
+            m0 = tm * BM;
+            n0 = tn * BN;
+        } else {
+            constexpr int SM = 128 / BM, SN = 256 / BN;  // the tiles of a 128 x 256 tile
+            tile_from_id(cp.id0 + cur / (SM * SN), p.tiles_m, p.tiles_n, tm, tn);
+            m0 = tm * 128 + cur % (SM * SN) / SN * BM;
+            n0 = tn * 256 + cur % SN * BN;
+        }
 #pragma unroll
         for (int e = 0; e < XDMA; ++e)
-            xoff[e] = min(m0 + 8 * wave + 64 * e + lane / 8, p.t - 1) * static_cast<int>(p.ld_x) + 16 * chunk;
+            xoff[e] = min(m0 + 8 * (wave + NW * e) + lane / 8, p.t - 1) * static_cast<int>(p.ld_x) + 16 * chunk;
 #pragma unroll
         for (int e = 0; e < WDMA; ++e)
-            woff[e] = min(n0 + 8 * wave + 64 * e + lane / 8, p.n - 1) * static_cast<int>(p.ld_w) + 16 * chunk;
+            woff[e] = min(n0 + 8 * wkb(e) + lane / 8, p.n - 1) * static_cast<int>(p.ld_w) + 16 * chunk;
         ws_off0 = min(n0 + colrel[0], p.n - 1) * static_cast<int>(p.ld_ws) * 4;
         ws_off1 = min(n0 + colrel[1], p.n - 1) * static_cast<int>(p.ld_ws) * 4;
-        // per 128: lane l % 16 of wave w loads the scale of tile row 16 w + l % 16 (clamped like the operands)
-        xs_off = min(m0 + 16 * wave + lane % 16, p.t - 1) * static_cast<int>(p.ld_xs) * 4;
+        // per 128: lane l % RW of wave w loads the scale of tile row RW w + l % RW (clamped like the operands)
+        xs_off = min(m0 + RW * wave + lane % RW, p.t - 1) * static_cast<int>(p.ld_xs) * 4;
     };
     set_tile();
     int ra[4], rb[4];
     {
-        const int rowa = wm * 64 + lane % 32, rowb = colrel[0];
+        const int rowa = wm * WR + lane % 32, rowb = colrel[0];
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             const int c = 2 * st + lane / 32;
@@ -629,18 +669,20 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
         float ws[2];
         float xs;  // per 128: the activation scale of this lane's staging row
     };
-    Set s0, s1, s2;  // group g's scales in set g mod 3
-    // the wave's loads of group g: its share of one operand's stage, then its two weight scales
+    Set sets[3];  // group g's scales in set g mod 3
+    // the wave's loads of group g: its share of one operand's stage, then its two weight scales (the load of one
+    // kilobyte is a lambda of plain values: a builtin whose arguments depend on the template's parameters is rejected on
+    // the host side, and hipcc then silently leaves out the kernel's host stub)
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    const auto load_kb = [&](const __amdgpu_buffer_rsrc_t res, lds_u32x4* dst, int off, int k0) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (lds_ptr)dst, 16, off, k0, 0, 0);
+    };
     const auto issue = [&](int g, lds_u32x4* xd, lds_u32x4* wd, Set& s) {
         const int k0 = g * 128;
 #pragma unroll
-        for (int e = 0; e < XDMA; ++e)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, (__attribute__((address_space(3))) void*)(xd + (wave + 8 * e) * 64), 16,
-                                                     xoff[e], k0, 0, 0);
+        for (int e = 0; e < XDMA; ++e) load_kb(xres, xd + (wave + NW * e) * 64, xoff[e], k0);
 #pragma unroll
-        for (int e = 0; e < WDMA; ++e)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, (__attribute__((address_space(3))) void*)(wd + (wave + 8 * e) * 64), 16,
-                                                     woff[e], k0, 0, 0);
+        for (int e = 0; e < WDMA; ++e) load_kb(wres, wd + wkb(e) * 64, woff[e], k0);
         s.ws[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsres, ws_off0, g * 4, 0));
         s.ws[1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsres, ws_off1, g * 4, 0));
         if constexpr (!PER_TOKEN)
@@ -650,9 +692,9 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
     // per 128: group g's scales (landed) from set s into their ring slot; the LDS write is complete on return
     const auto put_xs = [&](int g, const Set& s) __attribute__((always_inline)) {
         if constexpr (!PER_TOKEN) {
-            // every lane writes (lanes l, l + 16, l + 32, l + 48 the same value): no branch, which costs the kernel its
+            // every lane writes (lanes a multiple of RW apart the same value): no branch, which costs the kernel its
             // registers
-            lds_xs[(xb + g) & 3][16 * wave + lane % 16] = s.xs;
+            lds_xs[(xb + g) & 3][RW * wave + lane % RW] = s.xs;
             wait_vm_lgkm0<NLD>();
         }
     };
@@ -664,17 +706,17 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    float acc[2][2][16];
+    float acc[MBLK][2][16];
     const i32x16 zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    // int32 sums of the blocks in flight: block n = 4 g + b (group g, block b) in T[n mod 3] (with three groups a turn
-    // the index is a constant: (4 (g mod 3) + b) mod 3)
+    // int32 sums of the blocks in flight: block n = NB g + b (group g, block b) in T[n mod NT] (with three groups a turn the
+    // index is a constant: (NB (g mod 3) + b) mod NT)
     // Per 128 the links run one block behind (two buffers, index n mod 2): each link also reads 16 activation scales,
     // and beside a third buffer's 16 registers the SwiGLU -> int8 form spilled 44 registers and took 1.77 against
     // 1.52 ms at C4's gate/up (the down multiply ran alike both ways). The block's four MFMAs are issued before its
     // link, so the converts still find the previous block's sums complete.
     constexpr int NT = PER_TOKEN ? 3 : 2, LAG = NT - 1;
     i32x16 T[NT];
-    u32x4 a[2][4], b[2][4];
+    u32x4 a[MBLK][4], b[2][4];
     // one link: per token acc = f ws (first group) or fma(f, ws, acc); per 128 the scale is ws x xs of the output's
     // row in group g (the cpu-q8 chain, as gemm_big's)
     const auto link = [&](const i32x16& S, int i, int q, float ws, bool first, int g) {
@@ -685,7 +727,7 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
                 acc[i][q][r] = first ? __fmul_rn(f, ws) : __builtin_fmaf(f, ws, acc[i][q][r]);
             }
         } else {
-            const float* xr = lds_xs[(xb + g) & 3] + wm * 64 + i * 32 + 4 * (lane / 32);
+            const float* xr = lds_xs[(xb + g) & 3] + wm * WR + i * 32 + 4 * (lane / 32);
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
                 const float4 x4 = *reinterpret_cast<const float4*>(xr + 8 * r4);
@@ -701,18 +743,20 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
         }
     };
 
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
     // L(g), stage j = g mod 3: group g + 2's loads (clamped: past the end they repeat into stages nothing reads again,
     // so the wait counts stay exact) into the stage and scale set of group g - 1, then group g's 16 fragments; the
     // reads are complete before the barrier
     const auto slot_l = [&](int g, auto jt) __attribute__((always_inline)) {
         constexpr int j = decltype(jt)::value;
-        Set& nxt = j == 0 ? s2 : (j == 1 ? s0 : s1);
-        const Set& following = j == 0 ? s1 : (j == 1 ? s2 : s0);  // group g + 1's
+        const Set& following = sets[(j + 1) % 3];  // group g + 1's
         issue(min(g + 2, groups - 1), xstage(std::integral_constant<int, (j + 2) % 3>{}),
-              wstage(std::integral_constant<int, (j + 2) % 3>{}), nxt);
+              wstage(std::integral_constant<int, (j + 2) % 3>{}), sets[(j + 2) % 3]);
         __builtin_amdgcn_sched_barrier(0);
-        const lds_u32x4* tx = xstage(std::integral_constant<int, j>{});
-        const lds_u32x4* tw = wstage(std::integral_constant<int, j>{});
+        const lds_u32x4* tx = xstage(jt);
+        const lds_u32x4* tw = wstage(jt);
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             a[0][st] = tx[ra[st]];
@@ -720,7 +764,7 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
         }
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
-            a[1][st] = tx[ra[st] + 256];
+            if constexpr (MBLK > 1) a[MBLK - 1][st] = tx[ra[st] + 256];
             b[1][st] = tw[rb[st] + 512];
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -743,34 +787,32 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
         // multiply); 2: later groups
         constexpr int pmode = decltype(prev_t)::value;
         constexpr bool first = pmode == 0;
-        Set& cur = j == 0 ? s0 : (j == 1 ? s1 : s2);
-        const float gws0 = cur.ws[0], gws1 = cur.ws[1];
+        const float gws0 = sets[j].ws[0], gws1 = sets[j].ws[1];
 #pragma unroll
-        for (int blk = 0; blk < 4; ++blk) {
+        for (int blk = 0; blk < NB; ++blk) {
             const int i = blk / 2, q = blk % 2;
-            i32x16& S = T[(4 * j + blk) % NT];
+            i32x16& S = T[(NB * j + blk) % NT];
 #pragma unroll
             for (int st = 0; st < 4; ++st) S = mfma_i8_32(a[i][st], b[q][st], st == 0 ? zero16 : S);
             if (blk >= LAG) {
                 const int pb = blk - LAG;  // this group's block pb
-                link(T[(4 * j + pb) % NT], pb / 2, pb % 2, pb % 2 == 0 ? gws0 : gws1, first, g);
+                link(T[(NB * j + pb) % NT], pb / 2, pb % 2, pb % 2 == 0 ? gws0 : gws1, first, g);
             } else if constexpr (pmode > 0) {
-                const int pb = blk + 4 - LAG;  // the previous group's block pb
-                link(T[(4 * j + blk + NT - LAG) % NT], pb / 2, pb % 2, pb % 2 == 0 ? pw0 : pw1, pmode == 1, g - 1);
+                const int pb = blk + NB - LAG;  // the previous group's block pb
+                link(T[(NB * j + blk + NT - LAG) % NT], pb / 2, pb % 2, pb % 2 == 0 ? pw0 : pw1, pmode == 1, g - 1);
             }
         }
         pw0 = gws0;
         pw1 = gws1;
-        barrier();
+        // without the alternation the next L slot may follow at once: its loads go to a stage whose reads every wave
+        // completed before the last barrier
+        if constexpr (PP) barrier();
     };
 
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
     // a tile's first loads: groups 0 and 1 in stages and scale sets 0 and 1
     const auto first_loads = [&]() __attribute__((always_inline)) {
-        issue(0, xstage(I0{}), wstage(I0{}), s0);
-        issue(min(1, groups - 1), xstage(I1{}), wstage(I1{}), s1);
+        issue(0, xstage(I0{}), wstage(I0{}), sets[0]);
+        issue(min(1, groups - 1), xstage(I1{}), wstage(I1{}), sets[1]);
     };
     first_loads();
     // Tile loop. Per tile the barriers balance (group A: 1 + 2 groups + 1, group B: 1 + 1 + 2 groups); after the last
@@ -780,13 +822,13 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
     // there the next tile's loads follow it.
     for (;;) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MBLK; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
         wait_vm_lgkm0<NLD>();  // group 0's loads
-        put_xs(0, s0);
+        put_xs(0, sets[0]);
         barrier();
         if (group_b) barrier();  // B runs one slot behind A
         // group g in stage and scale set g mod 3; M of group 0 and group 1 by their own modes, then three groups a turn
@@ -814,13 +856,13 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
             slot_l(g + 1, I0{});
             slot_m(g + 1, I0{}, I2{});
         }
-        if (!group_b) barrier();  // matches group B's extra barrier
+        if (PP && !group_b) barrier();  // matches group B's extra barrier
         // the last group's last LAG blocks (group groups - 1, stage index (groups - 1) mod 3)
         const auto last_links = [&](auto jt) __attribute__((always_inline)) {
             constexpr int j = decltype(jt)::value;
 #pragma unroll
-            for (int pb = 4 - LAG; pb < 4; ++pb)
-                link(T[(4 * j + pb) % NT], pb / 2, pb % 2, pb % 2 == 0 ? pw0 : pw1, groups == 1, groups - 1);
+            for (int pb = NB - LAG; pb < NB; ++pb)
+                link(T[(NB * j + pb) % NT], pb / 2, pb % 2, pb % 2 == 0 ? pw0 : pw1, groups == 1, groups - 1);
         };
         switch ((groups - 1) % 3) {
         case 0: last_links(I0{}); break;
@@ -835,7 +877,7 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
         xb = (xb + groups) & 3;  // the next tile's group 0 takes the ring slot after this tile's last group
         if constexpr (EP == kSwigluQ8) {
             __syncthreads();
-            chain_epilogue<EP, YT, PER_TOKEN>(p, acc, mc, nc, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
+            chain_epilogue<EP, YT, PER_TOKEN, WM, WN, MBLK>(p, acc, mc, nc, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
             __syncthreads();  // weight stage 0 (the epilogue's scratch) is free again
             if (!more) break;
             set_tile();
@@ -845,7 +887,7 @@ __global__ void __launch_bounds__(512) gemm_chain(const ChainParams cp) {
                 set_tile();
                 first_loads();
             }
-            chain_epilogue<EP, YT, PER_TOKEN>(p, acc, mc, nc, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
+            chain_epilogue<EP, YT, PER_TOKEN, WM, WN, MBLK>(p, acc, mc, nc, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
             if (!more) break;
         }
     }
@@ -1071,6 +1113,89 @@ inline int device_cus() {
     return cus;
 }
 
+// The tile of a gemm_chain launch: WM x WN waves of 32 MBLK rows x 64 columns.
+struct ChainTile {
+    int wm, wn, mblk;
+    int per_cu;                // blocks a CU holds at once
+    double step[2], step2[2];  // us per group with one block on the CU, and with per_cu (per token, per 128)
+    double round[2];           // us per tile round besides (prologue, epilogue)
+    int rows() const { return 32 * mblk * wm; }
+    int cols() const { return 64 * wn; }
+    // us of `tiles` tiles: full rounds of per_cu blocks per CU, and a last one that may hold one block per CU
+    double cost(int tiles, int groups, int cus, bool per128) const {
+        const int slots = per_cu * cus, full = tiles / slots, rest = tiles % slots;
+        const int i = per128 ? 1 : 0;
+        return full * (groups * step2[i] + round[i]) + (rest == 0 ? 0.0 : groups * (rest <= cus ? step[i] : step2[i]) + round[i]);
+    }
+};
+
+// Which tile. Large problems take the 128 x 256 tile: the most outputs per operand byte and per instruction. Where its
+// grid leaves CUs idle (a narrow N, a last round with few tiles), smaller tiles of the same kernel fill them; every
+// output keeps its links' order, so the bits do not depend on the tile. The times below are fitted to forced-tile runs at
+// 19456 x 2560, 2560 x 9728, 2560 x 2560 and 7168 x 1024, T 65 .. 4096 (e.g. 2560 x 9728 per token, us: T = 300 128 x 256 80,
+// 128 x 128 56, 96 x 128 52, 64 x 128 46, 32 x 128 38; T = 896 82, 56, 54, 85, 94; T = 4096 171, 175, 209, 208, 300). A
+// step of a small tile is not a share of the large one's: each wave's converts and multiply-adds, its loads' issue and
+// the barrier remain.
+constexpr ChainTile kChain128x256{2, 4, 2, 1, {1.05, 1.45}, {1.05, 1.45}, {6.0, 7.0}};
+constexpr ChainTile kChain128x128{4, 2, 1, 1, {0.68, 0.80}, {0.68, 0.80}, {4.0, 5.0}};
+constexpr ChainTile kChain96x128{3, 2, 1, 1, {0.61, 0.82}, {0.61, 0.82}, {4.0, 4.0}};
+constexpr ChainTile kChain64x128{2, 2, 1, 2, {0.49, 0.62}, {1.07, 1.18}, {3.5, 3.5}};
+constexpr ChainTile kChain32x128{1, 2, 1, 2, {0.41, 0.68}, {0.73, 0.77}, {3.5, 3.0}};
+// the SwiGLU -> int8 epilogue needs 256 columns (one block of 128 outputs)
+constexpr ChainTile kChainQ8_128x256{2, 4, 2, 1, {1.70, 1.70}, {1.70, 1.70}, {9.0, 9.0}};
+constexpr ChainTile kChainQ8_64x256{2, 4, 1, 1, {0.95, 1.15}, {0.95, 1.15}, {6.0, 7.0}};
+
+struct ChainPlan {
+    int full;             // 128 x 256 tiles of the first launch (whole rounds; 0: none)
+    const ChainTile* tile;  // of everything, or of what the first launch leaves
+};
+
+inline ChainPlan chain_plan(int t, int n, int groups, bool q8_out, bool per128, int cus) {
+    const ChainTile& big = q8_out ? kChainQ8_128x256 : kChain128x256;
+    static const ChainTile* const plain[] = {&kChain128x128, &kChain96x128, &kChain64x128, &kChain32x128};
+    static const ChainTile* const fused[] = {&kChainQ8_64x256};
+    const ChainTile* const* small = q8_out ? fused : plain;
+    const int count = q8_out ? 1 : 4;
+    const int tiles = (t + 127) / 128 * ((n + 255) / 256), full = tiles / cus * cus;
+    ChainPlan best{0, &big};
+    double us = big.cost(tiles, groups, cus, per128);
+    for (int i = 0; i < count; ++i) {
+        const ChainTile& c = *small[i];
+        const double whole = c.cost((t + c.rows() - 1) / c.rows() * ((n + c.cols() - 1) / c.cols()), groups, cus, per128);
+        if (whole < 0.96 * us) us = whole, best = ChainPlan{0, &c};
+        if (full == 0 || full == tiles || 128 % c.rows() != 0) continue;
+        // whole rounds of the large tile, then the rest in small ones (a second launch, which starts when the slowest
+        // block of the first has ended: 6 us)
+        const double mixed = big.cost(full, groups, cus, per128) + 6.0 +
+                             c.cost((tiles - full) * (128 / c.rows()) * (256 / c.cols()), groups, cus, per128);
+        if (mixed < 0.96 * us) us = mixed, best = ChainPlan{full, &c};
+    }
+    return best;
+}
+
+// One launch of gemm_chain, persistent: at most per_cu blocks per CU, a whole number of blocks per XCD (the kernel's stride
+// through its XCD's tiles is grid / 8, so it must be at least 1; blocks whose range is empty leave at once). first, count:
+// the 128 x 256 tiles it covers (count 0: the whole problem on its own grid).
+template <int EP, int YT, bool PT, int WM, int WN, int MBLK>
+void launch_chain(ChainParams cp, int per_cu, int first, int count, hipStream_t stream) {
+    constexpr int BM = 32 * MBLK * WM, BN = 64 * WN;
+    if (count > 0) {
+        cp.p.tiles_m = (cp.p.t + 127) / 128;
+        cp.p.tiles_n = (cp.p.n + 255) / 256;
+        cp.id0 = first;
+        cp.total = count * (128 / BM) * (256 / BN);
+    } else {
+        cp.p.tiles_m = (cp.p.t + BM - 1) / BM;
+        cp.p.tiles_n = (cp.p.n + BN - 1) / BN;
+        cp.id0 = -1;
+        cp.total = cp.p.tiles_m * cp.p.tiles_n;
+    }
+    const int grid = 8 * std::max(1, std::min((cp.total + 7) / 8, per_cu * device_cus() / 8));
+    if (grid % 8 != 0 || grid < 8) throw LaunchError("gemm_q8: persistent grid must be a positive multiple of 8");
+    gemm_chain<EP, YT, PT, WM, WN, MBLK><<<dim3(grid), dim3(64 * WM * WN), 0, stream>>>(cp);
+    check_launch("gemm_q8 large-M kernel launch");
+}
+
 template <int EP, int YT, bool PT, int MODE>
 void launch_big(const GemmArgs& a, hipStream_t stream) {
     Params p = make_params(a);
@@ -1082,15 +1207,22 @@ void launch_big(const GemmArgs& a, hipStream_t stream) {
     const std::size_t lim = std::size_t{1} << 31;
     if constexpr (MODE == MODE_CHAIN) {
         if (x_bytes < lim && w_bytes < lim && ws_bytes < lim && xs_bytes < lim) {
-            const ChainParams cp{p, static_cast<unsigned>(x_bytes), static_cast<unsigned>(w_bytes),
+            const ChainParams cp{p, 0, -1, static_cast<unsigned>(x_bytes), static_cast<unsigned>(w_bytes),
                                  static_cast<unsigned>(ws_bytes), static_cast<unsigned>(xs_bytes)};
-            // persistent: at most one block per CU, a whole number of blocks per XCD (the kernel's stride through its
-            // XCD's tiles is grid / 8, so it must be at least 1; blocks whose range is empty leave at once)
-            const int tiles = p.tiles_m * p.tiles_n;
-            const int grid = 8 * std::max(1, std::min((tiles + 7) / 8, device_cus() / 8));
-            if (grid % 8 != 0 || grid < 8) throw LaunchError("gemm_q8: persistent grid must be a positive multiple of 8");
-            gemm_chain<EP, YT, PT><<<dim3(grid), dim3(512), 0, stream>>>(cp);
-            check_launch("gemm_q8 large-M kernel launch");
+            const ChainPlan plan = chain_plan(p.t, p.n, p.k / 128, EP == kSwigluQ8, !PT, device_cus());
+            const int tiles = p.tiles_m * p.tiles_n, rest = plan.full > 0 ? tiles - plan.full : 0;
+            if (plan.full > 0) launch_chain<EP, YT, PT, 2, 4, 2>(cp, 1, 0, plan.full, stream);
+            const ChainTile& c = *plan.tile;
+            if constexpr (EP == kSwigluQ8) {
+                if (c.mblk == 1) launch_chain<EP, YT, PT, 2, 4, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else launch_chain<EP, YT, PT, 2, 4, 2>(cp, c.per_cu, plan.full, rest, stream);
+            } else {
+                if (c.mblk == 2) launch_chain<EP, YT, PT, 2, 4, 2>(cp, c.per_cu, plan.full, rest, stream);
+                else if (c.wm == 4) launch_chain<EP, YT, PT, 4, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else if (c.wm == 3) launch_chain<EP, YT, PT, 3, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else if (c.wm == 2) launch_chain<EP, YT, PT, 2, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else launch_chain<EP, YT, PT, 1, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+            }
             return;
         }
     }
