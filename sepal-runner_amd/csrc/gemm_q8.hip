@@ -518,6 +518,53 @@ __global__ void __launch_bounds__(512) gemm_big(const Params p) {
     chain_epilogue<EP, YT, PER_TOKEN, 2, 4, 2, PER_TOKEN && MODE == MODE_CHAIN>(p, acc, m0, n0, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
 }
 
+// gemm_s8's epilogue of a tile: y = (float(S) * sx[t]) * sw[n], float32 or binary16 (round to nearest even); acc holds
+// float(S).
+template <int YT, int WM, int WN, int MBLK>
+__device__ __forceinline__ void s8_epilogue(const Params& p, float (&acc)[MBLK][2][16], int m0, int n0, int wm, int wn, int lane,
+                                            const int (&col)[2]) {
+    constexpr int WR = 32 * MBLK;
+    constexpr unsigned ES = YT == SEPAL_HIP_F16 ? 2 : 4;
+    const auto store = [](char* dst, float v) __attribute__((always_inline)) {
+        if constexpr (YT == SEPAL_HIP_F16) *reinterpret_cast<unsigned short*>(dst) = f32_to_f16_bits(v);
+        else *reinterpret_cast<float*>(dst) = v;
+    };
+    float sw[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) sw[q] = p.ws[static_cast<std::size_t>(min(col[q], p.n - 1)) * p.ld_ws];
+    char* const yb = static_cast<char*>(p.y);
+    if (m0 + WR * WM <= p.t && n0 + 64 * WN <= p.n) {
+        // a whole tile: no bounds checks; wave-uniform row and column bases, 32-bit lane offsets
+        const int wmu = __builtin_amdgcn_readfirstlane(wm), wnu = __builtin_amdgcn_readfirstlane(wn);
+        const unsigned lrow = 4u * static_cast<unsigned>(lane / 32);
+        const unsigned voff = (lrow * static_cast<unsigned>(p.ld_y) + lane % 32) * ES;
+        const unsigned xoff = lrow * static_cast<unsigned>(p.ld_xs) * 4u;
+#pragma unroll
+        for (int i = 0; i < MBLK; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const std::size_t row = static_cast<std::size_t>(m0 + wmu * WR + i * 32 + 8 * (r / 4) + (r % 4));
+                const float sx = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p.xs + row * p.ld_xs) + xoff);
+                char* const rp = yb + (row * p.ld_y + n0 + 128 * (wnu / 2) + 32 * (wnu % 2)) * ES;
+#pragma unroll
+                for (int q = 0; q < 2; ++q) store(rp + 64 * q * ES + voff, __fmul_rn(__fmul_rn(acc[i][q][r], sx), sw[q]));
+            }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < MBLK; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = m0 + wm * WR + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
+            if (row >= p.t) continue;
+            const float sx = p.xs[static_cast<std::size_t>(row) * p.ld_xs];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                if (col[q] < p.n)
+                    store(yb + (static_cast<std::size_t>(row) * p.ld_y + col[q]) * ES, __fmul_rn(__fmul_rn(acc[i][q][r], sx), sw[q]));
+        }
+}
+
 // ---- the chain, two wave groups in alternation (gemm_chain) ---------------------------------------------------------
 //
 // The 128 x 256 tile of gemm_big's chain mode: 8 waves of 64 x 64 outputs (2 x 2 blocks of MFMA 32x32x32 i8), K in
@@ -543,6 +590,10 @@ __global__ void __launch_bounds__(512) gemm_big(const Params p) {
 // read; every wave issues, reads and waits alike (only B's extra barrier at the start and A's at the end differ), so
 // the kernel has no branch between the groups' code. The launcher uses this kernel when every offset fits 32 bits.
 //
+// MODE_WHOLE / MODE_WHOLE_Y (gemm_s8, gemm_q8y): the same kernel without links, one int32 sum per output over the whole K
+// (exact in any order) and the K tail after the loop: 1024 x 7168 x 1024 25.6 -> 14.3 us, 1024 x 2560 x 4096 43.6 -> 20.7,
+// 65 x 2560 x 9728 75.4 -> 25.2 against gemm_big's form of it.
+//
 // Smaller tiles (WM x WN waves of 32 MBLK rows x 64 columns; chain_plan below picks) fill the chip where the 128 x 256
 // grid cannot. Eight waves alternate as above; blocks of 2, 4 or 6 waves run L(g), a barrier, M(g) and go straight on to
 // L(g + 1). At 2560 x 9728 (76 groups) a group takes 1.05 us on 128 x 256 tiles, 0.68 on 128 x 128, 0.61 on 96 x 128, 0.49 on
@@ -558,15 +609,17 @@ struct ChainParams {
     unsigned x_bytes, w_bytes, ws_bytes, xs_bytes;  // extents of X, W and their scales (buffer ranges)
 };
 
-template <int EP, int YT, bool PER_TOKEN, int WM, int WN, int MBLK>
+template <int EP, int YT, bool PER_TOKEN, int MODE, int WM, int WN, int MBLK>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM * WN == 2 ? 1 : 2))) gemm_chain(const ChainParams cp) {
     const Params& p = cp.p;
     constexpr int NW = WM * WN, WR = 32 * MBLK, BM = WR * WM, BN = 64 * WN, NB = 2 * MBLK;
     constexpr bool PP = NW == 8;  // two wave groups in alternation
+    constexpr bool WHOLE = MODE == MODE_WHOLE || MODE == MODE_WHOLE_Y;  // one int32 sum over the whole K, no links
+    static_assert(MODE != MODE_SUMS && (!WHOLE || (PER_TOKEN && EP != kSwigluQ8)), "modes");
     constexpr int RW = BM / NW;   // per 128: tile rows whose activation scale a wave loads
     // a wave's loads per group: its operand shares (1 KB each; with 6 waves the last of the weights' turn repeats), its
     // 2 weight scales and, per 128, one activation scale
-    constexpr int XDMA = BM / 8 / NW, WDMA = (BN / 8 + NW - 1) / NW, NLD = XDMA + WDMA + 2 + (PER_TOKEN ? 0 : 1);
+    constexpr int XDMA = BM / 8 / NW, WDMA = (BN / 8 + NW - 1) / NW, NLD = XDMA + WDMA + (WHOLE ? 0 : 2) + (PER_TOKEN ? 0 : 1);
     static_assert(XDMA * NW * 8 == BM && RW * NW == BM && RW <= 64, "whole shares");
     __shared__ __align__(1024) u32x4 lx0[BM * 8], lx1[BM * 8], lx2[BM * 8];
     __shared__ __align__(1024) u32x4 lw0[BN * 8], lw1[BN * 8], lw2[BN * 8];
@@ -683,8 +736,10 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
         for (int e = 0; e < XDMA; ++e) load_kb(xres, xd + (wave + NW * e) * 64, xoff[e], k0);
 #pragma unroll
         for (int e = 0; e < WDMA; ++e) load_kb(wres, wd + wkb(e) * 64, woff[e], k0);
-        s.ws[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsres, ws_off0, g * 4, 0));
-        s.ws[1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsres, ws_off1, g * 4, 0));
+        if constexpr (!WHOLE) {
+            s.ws[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsres, ws_off0, g * 4, 0));
+            s.ws[1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wsres, ws_off1, g * 4, 0));
+        }
         if constexpr (!PER_TOKEN)
             s.xs = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xsres, xs_off, (g >> p.act_shift) * 4, 0));
     };
@@ -707,6 +762,7 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
     };
 
     float acc[MBLK][2][16];
+    i32x16 tot[MBLK][2];  // WHOLE: the running int32 sums
     const i32x16 zero16 = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     // int32 sums of the blocks in flight: block n = NB g + b (group g, block b) in T[n mod NT] (with three groups a turn the
     // index is a constant: (NB (g mod 3) + b) mod NT)
@@ -791,6 +847,11 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int blk = 0; blk < NB; ++blk) {
             const int i = blk / 2, q = blk % 2;
+            if constexpr (WHOLE) {
+#pragma unroll
+                for (int st = 0; st < 4; ++st) tot[i][q] = mfma_i8_32(a[i][st], b[q][st], tot[i][q]);
+                continue;
+            }
             i32x16& S = T[(NB * j + blk) % NT];
 #pragma unroll
             for (int st = 0; st < 4; ++st) S = mfma_i8_32(a[i][st], b[q][st], st == 0 ? zero16 : S);
@@ -827,6 +888,10 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        if constexpr (WHOLE) {
+#pragma unroll
+            for (int i = 0; i < MBLK; ++i) tot[i][0] = tot[i][1] = zero16;
+        }
         wait_vm_lgkm0<NLD>();  // group 0's loads
         put_xs(0, sets[0]);
         barrier();
@@ -864,20 +929,72 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
             for (int pb = NB - LAG; pb < NB; ++pb)
                 link(T[(NB * j + pb) % NT], pb / 2, pb % 2, pb % 2 == 0 ? pw0 : pw1, groups == 1, groups - 1);
         };
-        switch ((groups - 1) % 3) {
-        case 0: last_links(I0{}); break;
-        case 1: last_links(I1{}); break;
-        default: last_links(I2{}); break;
+        if constexpr (!WHOLE) {
+            switch ((groups - 1) % 3) {
+            case 0: last_links(I0{}); break;
+            case 1: last_links(I1{}); break;
+            default: last_links(I2{}); break;
+            }
         }
         wait_vm_lgkm0<0>();  // this wave's repeated loads of the last groups have landed
         const int mc = m0, nc = n0;
         const int col[2] = {nc + colrel[0], nc + colrel[1]};
+        if constexpr (WHOLE) {
+            // the last K % 128 values (a multiple of 16): each lane loads its fragment chunks straight from global memory
+            // (rows clamped as above, chunks at or past K read as zero) and the MFMAs add them to the int32 sums
+            const int k0 = groups * 128, tail = p.k - k0;
+#pragma unroll
+            for (int st = 0; st < 4; ++st) {
+                if (32 * st >= tail) break;
+                const int c = 2 * st + lane / 32;
+                const bool in = 16 * c < tail;
+                u32x4 ta[MBLK], tb[2];
+#pragma unroll
+                for (int i = 0; i < MBLK; ++i) {
+                    const int row = min(mc + wm * WR + i * 32 + lane % 32, p.t - 1);
+                    ta[i] = in ? *reinterpret_cast<const u32x4*>(p.x + static_cast<std::size_t>(row) * p.ld_x + k0 + 16 * c)
+                               : u32x4{0u, 0u, 0u, 0u};
+                }
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int row = min(col[q], p.n - 1);
+                    tb[q] = in ? *reinterpret_cast<const u32x4*>(p.w + static_cast<std::size_t>(row) * p.ld_w + k0 + 16 * c)
+                               : u32x4{0u, 0u, 0u, 0u};
+                }
+#pragma unroll
+                for (int i = 0; i < MBLK; ++i)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) tot[i][q] = mfma_i8_32(ta[i], tb[q], tot[i][q]);
+            }
+            // the sums as floats, times the feature's scale where that comes first (kernel_i8_y; gemm_s8 multiplies by the
+            // row's scale first, in its epilogue)
+            float sw[2] = {1.0f, 1.0f};
+            if constexpr (MODE == MODE_WHOLE_Y) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) sw[q] = p.ws[static_cast<std::size_t>(min(col[q], p.n - 1)) * p.ld_ws];
+            }
+#pragma unroll
+            for (int i = 0; i < MBLK; ++i)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const float f = static_cast<float>(tot[i][q][r]);
+                        acc[i][q][r] = MODE == MODE_WHOLE_Y ? __fmul_rn(f, sw[q]) : f;
+                    }
+        }
+        const auto epilogue = [&]() __attribute__((always_inline)) {
+            if constexpr (MODE == MODE_WHOLE) s8_epilogue<YT, WM, WN, MBLK>(p, acc, mc, nc, wm, wn, lane, col);
+            else
+                chain_epilogue<EP, YT, PER_TOKEN, WM, WN, MBLK, PER_TOKEN && !WHOLE>(p, acc, mc, nc, wm, ib, hh, lane, tid, col,
+                                                                                    reinterpret_cast<float*>(lw0));
+        };
         cur += stride;
         const bool more = cur < hi;
         xb = (xb + groups) & 3;  // the next tile's group 0 takes the ring slot after this tile's last group
         if constexpr (EP == kSwigluQ8) {
             __syncthreads();
-            chain_epilogue<EP, YT, PER_TOKEN, WM, WN, MBLK>(p, acc, mc, nc, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
+            epilogue();
             __syncthreads();  // weight stage 0 (the epilogue's scratch) is free again
             if (!more) break;
             set_tile();
@@ -887,7 +1004,7 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
                 set_tile();
                 first_loads();
             }
-            chain_epilogue<EP, YT, PER_TOKEN, WM, WN, MBLK>(p, acc, mc, nc, wm, ib, hh, lane, tid, col, reinterpret_cast<float*>(lw0));
+            epilogue();
             if (!more) break;
         }
     }
@@ -1145,17 +1262,28 @@ constexpr ChainTile kChain32x128{1, 2, 1, 2, {0.41, 0.68}, {0.73, 0.77}, {3.5, 3
 constexpr ChainTile kChainQ8_128x256{2, 4, 2, 1, {1.70, 1.70}, {1.70, 1.70}, {9.0, 9.0}};
 constexpr ChainTile kChainQ8_64x256{2, 4, 1, 1, {0.95, 1.15}, {0.95, 1.15}, {6.0, 7.0}};
 
+// Whole-K sums (gemm_s8, gemm_q8y): no links.
+constexpr ChainTile kWhole128x256{2, 4, 2, 1, {0.80, 0.80}, {0.80, 0.80}, {6.0, 6.0}};
+constexpr ChainTile kWhole128x128{4, 2, 1, 1, {0.55, 0.55}, {0.55, 0.55}, {4.0, 4.0}};
+constexpr ChainTile kWhole96x128{3, 2, 1, 1, {0.50, 0.50}, {0.50, 0.50}, {4.0, 4.0}};
+constexpr ChainTile kWhole64x128{2, 2, 1, 2, {0.40, 0.40}, {0.70, 0.70}, {3.5, 3.5}};
+constexpr ChainTile kWhole32x128{1, 2, 1, 2, {0.35, 0.35}, {0.55, 0.55}, {3.5, 3.5}};
+enum { TILES_CHAIN = 0, TILES_INT8_OUT = 1, TILES_WHOLE = 2 };
+
 struct ChainPlan {
     int full;             // 128 x 256 tiles of the first launch (whole rounds; 0: none)
     const ChainTile* tile;  // of everything, or of what the first launch leaves
 };
 
-inline ChainPlan chain_plan(int t, int n, int groups, bool q8_out, bool per128, int cus) {
-    const ChainTile& big = q8_out ? kChainQ8_128x256 : kChain128x256;
-    static const ChainTile* const plain[] = {&kChain128x128, &kChain96x128, &kChain64x128, &kChain32x128};
-    static const ChainTile* const fused[] = {&kChainQ8_64x256};
-    const ChainTile* const* small = q8_out ? fused : plain;
-    const int count = q8_out ? 1 : 4;
+inline ChainPlan chain_plan(int t, int n, int groups, int kind, bool per128, int cus) {
+    static const ChainTile* const sets[3][5] = {
+        {&kChain128x256, &kChain128x128, &kChain96x128, &kChain64x128, &kChain32x128},
+        {&kChainQ8_128x256, &kChainQ8_64x256},
+        {&kWhole128x256, &kWhole128x128, &kWhole96x128, &kWhole64x128, &kWhole32x128},
+    };
+    const ChainTile& big = *sets[kind][0];
+    const ChainTile* const* small = sets[kind] + 1;
+    const int count = kind == TILES_INT8_OUT ? 1 : 4;
     const int tiles = (t + 127) / 128 * ((n + 255) / 256), full = tiles / cus * cus;
     ChainPlan best{0, &big};
     double us = big.cost(tiles, groups, cus, per128);
@@ -1176,7 +1304,7 @@ inline ChainPlan chain_plan(int t, int n, int groups, bool q8_out, bool per128, 
 // One launch of gemm_chain, persistent: at most per_cu blocks per CU, a whole number of blocks per XCD (the kernel's stride
 // through its XCD's tiles is grid / 8, so it must be at least 1; blocks whose range is empty leave at once). first, count:
 // the 128 x 256 tiles it covers (count 0: the whole problem on its own grid).
-template <int EP, int YT, bool PT, int WM, int WN, int MBLK>
+template <int EP, int YT, bool PT, int MODE, int WM, int WN, int MBLK>
 void launch_chain(ChainParams cp, int per_cu, int first, int count, hipStream_t stream) {
     constexpr int BM = 32 * MBLK * WM, BN = 64 * WN;
     if (count > 0) {
@@ -1192,7 +1320,7 @@ void launch_chain(ChainParams cp, int per_cu, int first, int count, hipStream_t 
     }
     const int grid = 8 * std::max(1, std::min((cp.total + 7) / 8, per_cu * device_cus() / 8));
     if (grid % 8 != 0 || grid < 8) throw LaunchError("gemm_q8: persistent grid must be a positive multiple of 8");
-    gemm_chain<EP, YT, PT, WM, WN, MBLK><<<dim3(grid), dim3(64 * WM * WN), 0, stream>>>(cp);
+    gemm_chain<EP, YT, PT, MODE, WM, WN, MBLK><<<dim3(grid), dim3(64 * WM * WN), 0, stream>>>(cp);
     check_launch("gemm_q8 large-M kernel launch");
 }
 
@@ -1205,23 +1333,25 @@ void launch_big(const GemmArgs& a, hipStream_t stream) {
     const std::size_t ws_bytes = MODE == MODE_CHAIN ? ((a.n - 1) * a.ld_s + a.k / 128) * 4 : 0;
     const std::size_t xs_bytes = MODE == MODE_CHAIN ? ((a.t - 1) * a.ld_xs + a.k / a.act_block) * 4 : 0;
     const std::size_t lim = std::size_t{1} << 31;
-    if constexpr (MODE == MODE_CHAIN) {
-        if (x_bytes < lim && w_bytes < lim && ws_bytes < lim && xs_bytes < lim) {
+    if constexpr (MODE != MODE_SUMS) {
+        // (a K below one group: gemm_big)
+        if (x_bytes < lim && w_bytes < lim && ws_bytes < lim && xs_bytes < lim && p.k >= 128) {
             const ChainParams cp{p, 0, -1, static_cast<unsigned>(x_bytes), static_cast<unsigned>(w_bytes),
                                  static_cast<unsigned>(ws_bytes), static_cast<unsigned>(xs_bytes)};
-            const ChainPlan plan = chain_plan(p.t, p.n, p.k / 128, EP == kSwigluQ8, !PT, device_cus());
+            const ChainPlan plan = chain_plan(p.t, p.n, p.k / 128, MODE == MODE_CHAIN ? (EP == kSwigluQ8 ? TILES_INT8_OUT : TILES_CHAIN) : TILES_WHOLE, !PT,
+                                              device_cus());
             const int tiles = p.tiles_m * p.tiles_n, rest = plan.full > 0 ? tiles - plan.full : 0;
-            if (plan.full > 0) launch_chain<EP, YT, PT, 2, 4, 2>(cp, 1, 0, plan.full, stream);
+            if (plan.full > 0) launch_chain<EP, YT, PT, MODE, 2, 4, 2>(cp, 1, 0, plan.full, stream);
             const ChainTile& c = *plan.tile;
             if constexpr (EP == kSwigluQ8) {
-                if (c.mblk == 1) launch_chain<EP, YT, PT, 2, 4, 1>(cp, c.per_cu, plan.full, rest, stream);
-                else launch_chain<EP, YT, PT, 2, 4, 2>(cp, c.per_cu, plan.full, rest, stream);
+                if (c.mblk == 1) launch_chain<EP, YT, PT, MODE, 2, 4, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else launch_chain<EP, YT, PT, MODE, 2, 4, 2>(cp, c.per_cu, plan.full, rest, stream);
             } else {
-                if (c.mblk == 2) launch_chain<EP, YT, PT, 2, 4, 2>(cp, c.per_cu, plan.full, rest, stream);
-                else if (c.wm == 4) launch_chain<EP, YT, PT, 4, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
-                else if (c.wm == 3) launch_chain<EP, YT, PT, 3, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
-                else if (c.wm == 2) launch_chain<EP, YT, PT, 2, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
-                else launch_chain<EP, YT, PT, 1, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                if (c.mblk == 2) launch_chain<EP, YT, PT, MODE, 2, 4, 2>(cp, c.per_cu, plan.full, rest, stream);
+                else if (c.wm == 4) launch_chain<EP, YT, PT, MODE, 4, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else if (c.wm == 3) launch_chain<EP, YT, PT, MODE, 3, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else if (c.wm == 2) launch_chain<EP, YT, PT, MODE, 2, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
+                else launch_chain<EP, YT, PT, MODE, 1, 2, 1>(cp, c.per_cu, plan.full, rest, stream);
             }
             return;
         }
