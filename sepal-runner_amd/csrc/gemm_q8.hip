@@ -240,6 +240,40 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[MBL
         }
         return;
     }
+    if (MBLK == 1 && p.ld_y < kEdgeMaxLd) {  // (beside the 128 x 256 tile's registers it spilled 14 to 30)
+        constexpr int ES = EP == SEPAL_HIP_SWIGLU && YT != SEPAL_HIP_F32 ? 2 : 4;
+        const int rows = min(BM, p.t - m0), ld = static_cast<int>(p.ld_y), width = EP == SEPAL_HIP_SWIGLU ? p.n / 2 : p.n;
+        const __amdgpu_buffer_rsrc_t yr = edge_buffer(static_cast<char*>(p.y) + static_cast<std::size_t>(m0) * p.ld_y * ES,
+                                                      (static_cast<long long>(rows - 1) * ld + width) * ES);
+        const int r0 = wm * WR + 4 * (lane / 32), f = n0 / 2 + 64 * ib + 32 * hh + lane % 32;
+#pragma unroll
+        for (int i = 0; i < MBLK; ++i) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four rows at a time: the offsets would take registers
+                const int row = r0 + i * 32 + 8 * (r / 4) + (r % 4);
+                float v0 = acc[i][0][r], v1 = acc[i][1][r];
+                if constexpr (PER_TOKEN) {
+                    const float xs = p.xs[static_cast<std::size_t>(m0 + min(row, rows - 1)) * p.ld_xs];
+                    v0 = __fmul_rn(v0, xs);
+                    v1 = __fmul_rn(v1, xs);
+                }
+                if constexpr (EP == SEPAL_HIP_SWIGLU) {
+                    edge_out<YT>(yr, row < rows && f < width ? (row * ld + f) * ES : kEdgeSkip, swiglu_q8<FAST_SILU>(v0, v1));
+                } else {
+                    const int o0 = row < rows && col[0] < width ? (row * ld + col[0]) * ES : kEdgeSkip;
+                    const int o1 = row < rows && col[1] < width ? (row * ld + col[1]) * ES : kEdgeSkip;
+                    if constexpr (EP == SEPAL_HIP_ADD) {
+                        v0 = __fadd_rn(edge_load32(yr, o0), v0);
+                        v1 = __fadd_rn(edge_load32(yr, o1), v1);
+                    }
+                    edge_store32(yr, o0, v0);
+                    edge_store32(yr, o1, v1);
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < MBLK; ++i) {
 #pragma unroll
@@ -548,6 +582,26 @@ __device__ __forceinline__ void s8_epilogue(const Params& p, float (&acc)[MBLK][
                 char* const rp = yb + (row * p.ld_y + n0 + 128 * (wnu / 2) + 32 * (wnu % 2)) * ES;
 #pragma unroll
                 for (int q = 0; q < 2; ++q) store(rp + 64 * q * ES + voff, __fmul_rn(__fmul_rn(acc[i][q][r], sx), sw[q]));
+            }
+        return;
+    }
+    if (p.ld_y < kEdgeMaxLd) {
+        const int rows = min(WR * WM, p.t - m0), ld = static_cast<int>(p.ld_y);
+        const __amdgpu_buffer_rsrc_t yr = edge_buffer(yb + static_cast<std::size_t>(m0) * p.ld_y * ES,
+                                                      (static_cast<long long>(rows - 1) * ld + p.n) * ES);
+        const int r0 = wm * WR + 4 * (lane / 32);
+#pragma unroll
+        for (int i = 0; i < MBLK; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four rows at a time: the offsets would take registers
+                const int row = r0 + i * 32 + 8 * (r / 4) + (r % 4);
+                const float sx = p.xs[static_cast<std::size_t>(m0 + min(row, rows - 1)) * p.ld_xs];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int off = row < rows && col[q] < p.n ? (row * ld + col[q]) * static_cast<int>(ES) : kEdgeSkip;
+                    edge_out<YT>(yr, off, __fmul_rn(__fmul_rn(acc[i][q][r], sx), sw[q]));
+                }
             }
         return;
     }
@@ -1165,6 +1219,30 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) g
                     char* const dst = yb + (row * p.ld_y + n0 + 64 * wnu + 32 * q) * ES + voff;
                     if constexpr (YT == SEPAL_HIP_F16) *reinterpret_cast<unsigned short*>(dst) = f32_to_f16_bits(v);
                     else *reinterpret_cast<float*>(dst) = v;
+                }
+            }
+        return;
+    }
+    if (p.ld_y < kEdgeMaxLd) {
+        constexpr int ES = YT == SEPAL_HIP_F16 ? 2 : 4;
+        const int rows = min(BM, p.t - m0), ld = static_cast<int>(p.ld_y), c0 = n0 + 64 * wn + lane % 32;
+        const __amdgpu_buffer_rsrc_t yr = edge_buffer(static_cast<char*>(p.y) + static_cast<std::size_t>(m0) * p.ld_y * ES,
+                                                      (static_cast<long long>(rows - 1) * ld + p.n) * ES);
+        const int r0 = wm * 32 * MB + 4 * (lane / 32);
+        float sw[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) sw[q] = p.ws[static_cast<std::size_t>(min(c0 + 32 * q, p.n - 1)) * p.ld_ws];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four rows at a time: the offsets would take registers
+                const int row = r0 + i * 32 + 8 * (r / 4) + (r % 4);
+                const float sx = p.xs[static_cast<std::size_t>(m0 + min(row, rows - 1)) * p.ld_xs];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int off = row < rows && c0 + 32 * q < p.n ? (row * ld + c0 + 32 * q) * ES : kEdgeSkip;
+                    edge_out<YT>(yr, off, __fmul_rn(__fmul_rn(static_cast<float>(tot[i][q][r]), sx), sw[q]));
                 }
             }
         return;
