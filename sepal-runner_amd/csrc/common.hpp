@@ -206,13 +206,14 @@ __device__ __forceinline__ void store_out(void* y, std::size_t idx, float v) {
 }
 
 // Stores of an edge tile (rows past T or columns past N in it) without branches: a buffer over the tile's live rows, in
-// which an offset at or past its extent is not stored (and loads zero). With a branch per output instead, a 128 x 256 tile's
+// which an offset at or past its extent is not stored (and loads zero); a tile without live rows makes no buffer (its extent
+// would be negative, which the hardware reads as nearly 4 GiB, past kEdgeSkip) and stores nothing. With a branch per output instead, a 128 x 256 tile's
 // stores took 7 us longer. The functions take plain values: a builtin whose arguments depend on template parameters is
 // rejected on the host side, and hipcc then leaves out the kernel's host stub.
 constexpr int kEdgeSkip = 0x7FFFFFF0;                     // an offset past every such buffer
 constexpr std::size_t kEdgeMaxLd = std::size_t{1} << 20;  // row strides below this: the offsets of 256 rows fit 31 bits
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t edge_buffer(void* base, long long bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes), 0x00020000);
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, static_cast<int>(bytes > 0 ? bytes : 0), 0x00020000);
 }
 __device__ __forceinline__ void edge_store32(const __amdgpu_buffer_rsrc_t r, int off, float v) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, off, 0, 0);

@@ -242,7 +242,9 @@ __device__ __forceinline__ void chain_epilogue(const Params& p, float (&acc)[MBL
     }
     if (MBLK == 1 && p.ld_y < kEdgeMaxLd) {  // (beside the 128 x 256 tile's registers it spilled 14 to 30)
         constexpr int ES = EP == SEPAL_HIP_SWIGLU && YT != SEPAL_HIP_F32 ? 2 : 4;
-        const int rows = min(BM, p.t - m0), ld = static_cast<int>(p.ld_y), width = EP == SEPAL_HIP_SWIGLU ? p.n / 2 : p.n;
+        const int rows = min(BM, p.t - m0);
+        if (rows <= 0) return;  // a split tile's part wholly past T: a buffer of no rows
+        const int ld = static_cast<int>(p.ld_y), width = EP == SEPAL_HIP_SWIGLU ? p.n / 2 : p.n;
         const __amdgpu_buffer_rsrc_t yr = edge_buffer(static_cast<char*>(p.y) + static_cast<std::size_t>(m0) * p.ld_y * ES,
                                                       (static_cast<long long>(rows - 1) * ld + width) * ES);
         const int r0 = wm * WR + 4 * (lane / 32), f = n0 / 2 + 64 * ib + 32 * hh + lane % 32;
@@ -587,6 +589,7 @@ __device__ __forceinline__ void s8_epilogue(const Params& p, float (&acc)[MBLK][
     }
     if (p.ld_y < kEdgeMaxLd) {
         const int rows = min(WR * WM, p.t - m0), ld = static_cast<int>(p.ld_y);
+        if (rows <= 0) return;  // a split tile's part wholly past T: a buffer of no rows
         const __amdgpu_buffer_rsrc_t yr = edge_buffer(yb + static_cast<std::size_t>(m0) * p.ld_y * ES,
                                                       (static_cast<long long>(rows - 1) * ld + p.n) * ES);
         const int r0 = wm * WR + 4 * (lane / 32);
@@ -1225,7 +1228,9 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) g
     }
     if (p.ld_y < kEdgeMaxLd) {
         constexpr int ES = YT == SEPAL_HIP_F16 ? 2 : 4;
-        const int rows = min(BM, p.t - m0), ld = static_cast<int>(p.ld_y), c0 = n0 + 64 * wn + lane % 32;
+        const int rows = min(BM, p.t - m0);
+        if (rows <= 0) return;  // a split tile's half wholly past T: a buffer of no rows
+        const int ld = static_cast<int>(p.ld_y), c0 = n0 + 64 * wn + lane % 32;
         const __amdgpu_buffer_rsrc_t yr = edge_buffer(static_cast<char*>(p.y) + static_cast<std::size_t>(m0) * p.ld_y * ES,
                                                       (static_cast<long long>(rows - 1) * ld + p.n) * ES);
         const int r0 = wm * 32 * MB + 4 * (lane / 32);

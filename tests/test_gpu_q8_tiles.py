@@ -28,9 +28,10 @@ def host(t):
     return t.cpu().numpy()
 
 
-# t, n, k (256 CUs): 32 x 128; 64 x 128; 96 x 128; 128 x 128; 128 x 256; one and two rounds of 128 x 256 and the rest small
+# t, n, k (256 CUs): 32 x 128; 64 x 128; 96 x 128; 128 x 128; 128 x 256; one and two rounds of 128 x 256 and the rest small;
+# a round of 128 x 256 and parts of the rest's tiles wholly past T
 SHAPES = [(65, 2560, 384), (300, 2576, 384), (450, 2560, 768), (897, 2560, 768), (1300, 2576, 768), (2100, 2560, 384),
-          (511, 19456, 2560), (900, 19456, 2560), (97, 128, 128), (66, 16, 256)]
+          (511, 19456, 2560), (900, 19456, 2560), (97, 128, 128), (66, 16, 256), (3872, 2560, 1280), (2200, 4352, 1280)]
 
 
 @pytest.mark.parametrize("act", ["token", "128"])

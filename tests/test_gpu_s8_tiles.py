@@ -17,9 +17,11 @@ def sm():
     return sepal_mlp
 
 
-# t, n, k (256 CUs): 32, 64, 96, 128 x 128 and 128 x 256 tiles; full rounds and a rest; one row; K under a group
+# t, n, k (256 CUs): 32, 64, 96, 128 x 128 and 128 x 256 tiles; full rounds and a rest; one row; K under a group;
+# parts of the rest's tiles wholly past T (sub-tiles of 128 x 256, halves of 256 x 256)
 SHAPES = [(65, 2560, 400), (33, 130, 144), (511, 2560, 1040), (640, 2574, 272), (1024, 2560, 1136), (1500, 2560, 528),
-          (2100, 2560, 256), (1024, 7168, 1024), (4096, 2560, 1152), (1, 34, 128), (70, 300, 112), (300, 514, 16)]
+          (2100, 2560, 256), (1024, 7168, 1024), (4096, 2560, 1152), (1, 34, 128), (70, 300, 112), (300, 514, 16),
+          (3872, 2560, 2560), (3104, 2574, 2560), (3104, 7168, 128)]
 
 
 @pytest.mark.parametrize("t,n,k", SHAPES)
