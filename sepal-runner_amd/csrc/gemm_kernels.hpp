@@ -163,6 +163,9 @@ struct MidGemmPlan {
 };
 bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan);
 void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStream_t stream);
+// The Store / Add multiply of a float32 X of up to 24 rows (N < 8192), from its hi and lo bf16 rows (pairs: hi [t, k], then lo [t, k]).
+bool mid_pairs_plan(const GemmArgs& a, MidGemmPlan& plan);
+void launch_mid_pairs(const GemmArgs& a, const MidGemmPlan& plan, const void* pairs, hipStream_t stream);
 // x bf16 [t, hidden] -> h binary16 [t, inter] -> part float32 [parts][t][hidden] -> y float32 [t, hidden] and, when
 // xn is set, xn bf16 [t, hidden] = RMSNorm(y) (cpu-q8 order, identity weight). stream_w: w_gu and w_d in the stream
 // layout (launch_stream_layout; the same bits).

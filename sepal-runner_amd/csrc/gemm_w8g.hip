@@ -1434,7 +1434,7 @@ void launch_big(const GemmArgs& a, hipStream_t stream) {
 
 // Whether a problem takes the small-M (weight-streaming) kernels: they write float32 (or SwiGLU outputs); a binary16
 // Store always takes the large-M kernels. By default they take T <= 32 with N < 8192 of what the kernels asked first
-// (dispatch_path) refuse, and of the two multiplies of a float32 X: measured on the model's weight
+// (dispatch_path; of a float32 X mid_pairs_plan) refuse: measured on the model's weight
 // shapes, the large-M kernels' small-grid plan (64-row blocks, K split) is faster above 32 rows (the streaming kernels
 // double their time from 33 rows, at 64-row tiles) and at any T for N >= 8192 (gate/up 19456 x 2560: 20 against
 // 24 us at T = 1), and the streaming kernels are faster for the narrow, long-K down shape (2560 x 9728: 22.5 against
@@ -1549,6 +1549,14 @@ void launch_f32(const GemmArgs& a, hipStream_t stream) {
     if (a.xsplit == nullptr) throw LaunchError("gemm_w8g: float32 X needs the split buffer");
     const int t = static_cast<int>(a.t), k = static_cast<int>(a.k);
     auto* pairs = static_cast<unsigned short*>(a.xsplit);
+    MidGemmPlan mid;
+    if (mid_pairs_plan(a, mid)) {
+        // few rows: hi and lo as the rows of one multiply, which reads the weights once; its planes are added in order
+        split_kernel<<<grid_for(a.t * (a.k / 8)), 256, 0, stream>>>(static_cast<const float*>(a.x), a.ld_x, pairs, t, k, 1);
+        check_launch("gemm_w8g split launch");
+        launch_mid_pairs(a, mid, pairs, stream);
+        return;
+    }
     if (!small_path(a) && big3_takes(a, 2 * a.k, 2 * a.k)) {
         // one pass of the 64-wide-step kernel over the hi + lo row (twice the MFMAs of a 16-bit X)
         split_kernel<<<grid_for(a.t * (a.k / 8)), 256, 0, stream>>>(static_cast<const float*>(a.x), a.ld_x, pairs, t, k, 0);

@@ -430,7 +430,9 @@ void launch_mt(const Params& p, int nt, std::size_t lds, hipStream_t stream) {
 
 } // namespace mid
 
-bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan) {
+namespace {
+
+bool make_plan(const GemmArgs& a, bool q8, int max_parts, MidGemmPlan& plan) {
     if (a.config >= 0 || a.t > kSmallM || a.w_stream || a.k % 128 != 0) return false;
     if (!q8 && a.x_type != SEPAL_HIP_BF16 && a.x_type != SEPAL_HIP_F16) return false;
     const bool swiglu = a.epilogue == SEPAL_HIP_SWIGLU;
@@ -450,7 +452,7 @@ bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan) {
     for (const int nt : {5, 3, 2}) {
         if (nt > max_nt) continue;
         const int spans = (tiles + nt - 1) / nt;
-        for (int kp = 1; kp <= 16 && (kp == 1 || (!swiglu && groups / kp >= 4)); ++kp) {
+        for (int kp = 1; kp <= max_parts && (kp == 1 || (!swiglu && groups / kp >= 4)); ++kp) {
             if (kp > 1 && static_cast<std::size_t>(kp) * a.t * a.n * sizeof(float) > kPartialBytes) break;
             const int gpt = (groups + kp - 1) / kp;
             // the kilobytes a CU streams (the groups of a part go to a SIMD's two waves, four SIMDs), and the parts' sum
@@ -467,7 +469,8 @@ bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan) {
     return true;
 }
 
-void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStream_t stream) {
+// The multiply alone: Y, or its K-parts [plan.parts][t][n] at part.
+void launch_multiply(const GemmArgs& a, bool q8, const MidGemmPlan& plan, float* part, hipStream_t stream) {
     mid::Params p{};
     const std::size_t xb = q8 ? 1 : 2;
     p.x = a.x;
@@ -482,8 +485,8 @@ void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStr
     p.xs = a.xs;
     p.ld_xs = a.ld_xs;
     const bool per128 = q8 && (a.act_block != a.k || a.k == 128);
-    p.y = a.y;
-    p.ld_y = a.ld_y;
+    p.y = part != nullptr ? static_cast<void*>(part) : a.y;
+    p.ld_y = part != nullptr ? a.n : a.ld_y;
     p.y_type = a.y_type;
     p.epilogue = a.epilogue;
     p.t = static_cast<int>(a.t);
@@ -492,12 +495,6 @@ void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStr
     p.tiles = static_cast<int>(a.n / 16);
     p.parts = plan.parts;
     p.spans = (p.tiles + plan.nt - 1) / plan.nt;
-    float* part = nullptr;
-    if (p.parts > 1) {
-        if (a.scratch == nullptr) throw LaunchError("mid-M multiply: scratch missing");
-        part = reinterpret_cast<float*>(static_cast<char*>(a.scratch) + kCounterBytes);
-        p.y = part;
-    }
     const int mt = p.t <= 32 ? 2 : (p.t <= 48 ? 3 : 4);
     const std::size_t gpt = (a.k / 128 + plan.parts - 1) / plan.parts;
     const std::size_t lds = per128 ? gpt * 16 * mt * sizeof(float) : 0;
@@ -505,8 +502,55 @@ void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStr
     else if (q8) mid::launch_mt<mid::kI8Token>(p, plan.nt, lds, stream);
     else if (a.x_type == SEPAL_HIP_BF16) mid::launch_mt<SEPAL_HIP_BF16>(p, plan.nt, lds, stream);
     else mid::launch_mt<SEPAL_HIP_F16>(p, plan.nt, lds, stream);
+}
+
+float* partial_zone(const GemmArgs& a) {
+    if (a.scratch == nullptr) throw LaunchError("mid-M multiply: scratch missing");
+    return reinterpret_cast<float*>(static_cast<char*>(a.scratch) + kCounterBytes);
+}
+
+// The multiply of the hi and lo rows of a float32 X as one of 2 T bf16 rows.
+GemmArgs pairs_args(const GemmArgs& a) {
+    GemmArgs b = a;
+    b.x_type = SEPAL_HIP_BF16;
+    b.ld_x = a.k;
+    b.t = 2 * a.t;
+    b.epilogue = SEPAL_HIP_STORE;
+    return b;
+}
+
+} // namespace
+
+bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan) { return make_plan(a, q8, 16, plan); }
+
+void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStream_t stream) {
+    float* const part = plan.parts > 1 ? partial_zone(a) : nullptr;
+    launch_multiply(a, q8, plan, part, stream);
     if (part != nullptr)
         launch_parts_add(plan.parts, a.epilogue == SEPAL_HIP_ADD, a.t, a.n, part, static_cast<float*>(a.y), a.ld_y, stream);
+}
+
+// A float32 X of up to 24 rows, N < 8192: its hi and lo rows are one multiply of up to 48 rows, which reads the weights
+// once, where two multiplies read them twice. Measured (us a call, graph replays over cold weights, the split included):
+// 2560 x 9728 at 1 / 16 / 24 rows 28.0 / 30.9 / 29.8 -> 16.2 / 19.0 / 21.3, 2560 x 4096 21.8 / 23.6 / 22.7 -> 11.7 / 13.8 /
+// 15.7, 1024 x 4096 19.1 / 20.6 / 16.8 -> 9.2 / 10.7 / 11.9; 1.1 to 2.2 times over N 1024 .. 8176, K 1024 .. 5120. At 25 to 32
+// rows (three tiles a block) 6656 x 5120 took 36.2 against 35.0; from N = 8192 the other route is one pass of the large-M
+// hi + lo form, and 10496 x 5120 took 36.6 against 30.8 at 17 rows. What bounds it: the split, the multiply and the sum are
+// three dependent launches around one pass over the weights. SwiGLU keeps its own route (the sum comes before the silu).
+bool mid_pairs_plan(const GemmArgs& a, MidGemmPlan& plan) {
+    if (a.x_type != SEPAL_HIP_F32 || a.epilogue == SEPAL_HIP_SWIGLU || a.t > 24 || a.n >= 8192) return false;
+    const GemmArgs b = pairs_args(a);
+    // (the sum takes 16 parts: hi and lo of up to 8)
+    return 2 * a.t * a.n * sizeof(float) <= kPartialBytes && make_plan(b, false, 8, plan);
+}
+
+void launch_mid_pairs(const GemmArgs& a, const MidGemmPlan& plan, const void* pairs, hipStream_t stream) {
+    GemmArgs b = pairs_args(a);
+    b.x = pairs;
+    float* const part = partial_zone(a);
+    launch_multiply(b, false, plan, part, stream);
+    // [parts][2 T][n]: each part's hi rows, then its lo rows, are two planes of [T][n]
+    launch_parts_add(2 * plan.parts, a.epilogue == SEPAL_HIP_ADD, a.t, a.n, part, static_cast<float*>(a.y), a.ld_y, stream);
 }
 
 } // namespace sepal::hip

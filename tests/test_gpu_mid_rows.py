@@ -107,3 +107,25 @@ def test_rows_do_not_see_each_other(sm, t):
     b = sm.gemm_w8g(x2, q, s)
     assert torch.equal(a[t // 2], b[t // 2])
     assert torch.isfinite(b[1:]).all() and not torch.isfinite(b[0]).any()
+
+
+# t, n, k: one row; one tile and one group; tiles short of a block; K-parts; both sides of 24 rows and of N = 8192
+@pytest.mark.parametrize("t,n,k", [(1, 16, 128), (5, 144, 384), (16, 2560, 9728), (17, 48, 640), (24, 2576, 1280),
+                                   (24, 8176, 256), (24, 256, 9728), (25, 2560, 1152), (24, 8192, 512)])
+def test_float32_x(sm, t, n, k):
+    """A float32 X up to 24 rows as its hi and lo bf16 rows in one multiply: hi + lo is within 2^-17 of x."""
+    print("[case] mid rows float32", t, n, k, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(t + n + k)
+    q, s = sm.quantize_group_s8((torch.randn(n, k, generator=g, device="cuda") * 0.02).half())
+    x = torch.randn(t, k + 4, generator=g, device="cuda")[:, :k]
+    deq = (q.double().view(n, k // 128, 128) * s.double()[:, :, None]).view(n, k)
+    ref, mag = x.double() @ deq.T, x.double().abs() @ deq.abs().T
+    u = (2 * k + k // 128 + 16) * 2.0**-24 + 2.0**-17
+    y = torch.full((t, n + 4), 7.0, device="cuda")
+    sm.gemm_w8g(x, q, s, y=y[:, :n])
+    _check(y[:, :n], ref, mag, u)
+    assert (y[:, n:] == 7.0).all()
+    first = y[:, :n].clone()
+    sm.gemm_w8g(x, q, s, y=y[:, :n], epilogue=sm.ADD)
+    _check(y[:, :n], 2 * ref, 2 * mag, u)
+    assert torch.equal(sm.gemm_w8g(x, q, s), first)
