@@ -120,11 +120,11 @@ SEPAL_HIP_API int32_t sepal_hip_quantize_rows_s8(const void* x, int32_t x_type, 
  * large-M path reproduces cpu-q8 bit for bit. act_block = K (one scale per token): y = (f_0 * ws_0, then
  * fma(f_b, ws_b, y)) * xs. Epilogues STORE / ADD / SWIGLU (silu with the cpu-q8 exp polynomial); Y float32
  * [T, ld_y], or y_type for SWIGLU. K a multiple of 128; strides multiples of 16; 16-byte aligned pointers. `config`
- * -1 takes a small-M path up to 64 rows (at T <= 16 with a float32 Y the M <= 16 stack's q8 passes where the shape
- * fits them, else a kernel that splits K over waves and blocks), 0 the large-M path, 1 the streaming small-M path,
- * 2 the streaming path with the chain whole; the small-M paths split K, which keeps the int32 group sums exact but adds
- * the splits' partial chains (within tolerance, not bit for bit); config 2 keeps the chain whole
- * (bit for bit).
+ * -1 has the bits of the small-M path up to 64 rows (above 32 rows only for N < 8192; at T <= 16 with a float32 Y the
+ * M <= 16 stack's q8 passes run where the shape fits them, with an order of their own) and of the large-M path
+ * otherwise; 0 forces the large-M path, 1 the streaming small-M path, 2 the streaming path with the chain whole; the
+ * small-M path splits K into runs, which keeps the int32 group sums exact but adds the runs' partial chains in order
+ * (within tolerance, not bit for bit); config 2 keeps the chain whole (bit for bit).
  * Replaces kernel_i8_z + finish_tile (runner/src/cpu/gemm_kernels_avx512.cpp:67-115, gemm.cpp:417-447, 545-569)
  * with per-group scales (the per-channel launch_gemm_s8 is sepal_hip_gemm_s8). */
 SEPAL_HIP_API int32_t sepal_hip_gemm_q8(const int8_t* xq, size_t ld_x, const float* xs, size_t ld_xs, size_t act_block,
@@ -199,7 +199,7 @@ SEPAL_HIP_API int32_t sepal_hip_gemm_w8a16(const void* x, size_t ld_x, const int
  * [T, ld_hq] (N/2 columns), hs float32 [T, ld_hs] (N/256 used); equal, bit for bit, to sepal_hip_gemm_q8 (SWIGLU,
  * float32 H) followed by sepal_hip_quantize_rows_s8 (block 128) on the same path. N a multiple of 256; other rules and
  * `config` as sepal_hip_gemm_q8. The large-M kernel quantizes in its epilogue (one tile holds one 128-column block);
- * the small-M path computes H into the workspace first. No single reference function: it fuses finish_tile's SwiGLU
+ * up to 64 rows a small-M kernel may compute H into the workspace first (the same bits). No single reference function: it fuses finish_tile's SwiGLU
  * (runner/src/cpu/gemm.cpp:417-447) with pack_acts (gemm.cpp:285-306), the SwiGLU -> int8 fusion the reference lists
  * as not done (runner/cuda/README.md:1513-1515). */
 SEPAL_HIP_API int32_t sepal_hip_gemm_q8_swiglu_quantize(const int8_t* xq, size_t ld_x, const float* xs, size_t ld_xs,

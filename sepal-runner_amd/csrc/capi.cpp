@@ -655,7 +655,14 @@ int32_t sepal_hip_gemm_q8_swiglu_quantize(const int8_t* xq, size_t ld_x, const f
         a.t = t;
         a.n = n;
         a.k = k;
-        const bool large = config == 0 || (config < 0 && t > kSmallM);
+        // (33-64 rows with N >= 8192: the same bits either way; the fused form where a graph is being captured, since it needs
+        // no workspace that would have to exist by then)
+        bool large = config == 0 || (config < 0 && t > kSmallM);
+        if (config < 0 && !large && !q8_streams(t, n)) {
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(st, &cap) != hipSuccess) throw LaunchError("gemm_q8_swiglu_quantize: hipStreamIsCapturing failed");
+            large = cap != hipStreamCaptureStatusNone;
+        }
         if (large) {
             a.y = hq;
             a.ld_y = ld_hq;
@@ -802,7 +809,7 @@ void check_stack_args(int32_t kind, size_t hidden, size_t inter, const void* x, 
     require(hidden < 0x7FFFFFFFu && inter < 0x7FFFFFFFu, "mlp_stack: dimension beyond 2^31");
 }
 
-StackZones stack_zones(int kind, std::size_t t, std::size_t hidden, std::size_t inter, std::size_t act_block) {
+StackZones stack_zones(int kind, std::size_t t, std::size_t hidden, std::size_t inter, std::size_t act_block, bool fuse_h) {
     StackZones z;
     z.per_token = act_block == 0;
     z.ab_h = z.per_token ? hidden : 128;
@@ -831,7 +838,7 @@ StackZones stack_zones(int kind, std::size_t t, std::size_t hidden, std::size_t 
     // general: H [t, inter] (binary16 for w8g and for q8 with one scale per token; float32 for kind 2, and for q8 per
     // 128 unless the gate/up epilogue quantizes it); q8 also the int8 layer input and int8 H with their scales; kind 2
     // the hi + lo pairs of H for the down multiply
-    z.fused_h = kind == 1 && z.ab_i == 128 && t > kSmallM;
+    z.fused_h = kind == 1 && z.ab_i == 128 && (t > kSmallM || (fuse_h && !q8_streams(t, 2 * inter)));
     const std::size_t h_bytes = kind == 0 ? t * inter * 2 : (z.fused_h ? 0 : t * inter * 4);
     z.off_qx = z.off_h + up256(h_bytes);
     z.off_sx = z.off_qx + (kind == 1 ? up256(t * hidden) : 0);
@@ -1083,6 +1090,8 @@ int32_t sepal_hip_mlp_stack_noalloc(int32_t kind, size_t layers, size_t t, size_
             z.img = z.img_dn = 0;
             z.end = z.off_img;
         }
+        // (without the float32 H of 33-64 rows per 128: its quantization in the gate/up epilogue, the same bits)
+        if (z.end > kStaticScratchBytes && kind == 1) z = stack_zones(kind, t, hidden, inter, act_block, true);
         require(z.end <= kStaticScratchBytes,
                 "mlp_stack_noalloc: this shape needs " + std::to_string(z.end) + " bytes of scratch, beyond the " +
                     std::to_string(kStaticScratchBytes) + " of the static scratch (call with fewer rows)");

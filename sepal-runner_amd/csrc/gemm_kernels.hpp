@@ -8,9 +8,9 @@ namespace sepal::hip {
 // Rows at or below which the multiplies take the weight-streaming small-M path.
 inline constexpr std::size_t kSmallM = 64;
 
-// Default routing of the q8 multiply (config -1) for what mid_gemm_plan refuses (offsets beyond 32 bits): the small-M
-// (streaming) kernels up to kSmallM rows, except above 32 rows with N >= 8192, where the large-M kernels are faster (gate/up 19456 x 2560 at T = 40-64: 28-30 against 41-43 us
-// per token, 35-37 against 43-44 per 128; 12288 x 2560: 29-33 against 35) and also bit-exact to cpu-q8.
+// Whose order of links the q8 multiply keeps by default (config -1) up to kSmallM rows: true, the small-M (streaming)
+// kernels' (runs of groups, stream_q8_order); false, the whole chain of the large-M kernels, cpu-q8 bit for bit. The
+// kernels themselves run what launch_q8_rows refuses.
 inline bool q8_streams(std::size_t t, std::size_t n) { return t <= kSmallM && (t <= 32 || n < 8192); }
 
 struct GemmArgs {
@@ -79,6 +79,20 @@ void launch_w8g_image(const std::int8_t* w, std::size_t ld_w, std::size_t n, std
 inline std::size_t gemm_w8g_split_bytes(const GemmArgs& a) { return (a.t * a.k * 4 + 255) / 256 * 256; }
 void launch_stream_w8g(const GemmArgs& a, hipStream_t stream);
 void launch_stream_q8(const GemmArgs& a, hipStream_t stream);
+// The order of links of launch_stream_q8: `splits` runs of `gps` groups (the last shorter), each a chain from +0, added in
+// order. Refuses (throws) what that kernel does not take.
+void stream_q8_order(const GemmArgs& a, int& splits, int& gps);
+// One q8 multiply of up to 64 rows (q8_small.hip; config -1), with the bits of the kernel that q8_streams names.
+// q8_rows_plan returns false for what the kernel does not take (another T or config, offsets beyond 32 bits, a run's scales
+// beyond the LDS).
+struct Q8RowsPlan {
+    bool whole;       // the whole chain (first product's sign kept)
+    int splits, gps;  // runs of gps groups
+    int parts, wt;    // blocks a tile's runs are spread over (1, or one per run); 16-row weight tiles of a block
+};
+bool q8_rows_blocks(int mt, bool per128, int tiles, int groups, int splits, int gps, int cus, Q8RowsPlan& plan);
+bool q8_rows_plan(const GemmArgs& a, Q8RowsPlan& plan);
+void launch_q8_rows(const GemmArgs& a, const Q8RowsPlan& plan, hipStream_t stream);
 void launch_gemm_q8(const GemmArgs& a, hipStream_t stream);
 // The int8-activation multiply with per-channel weight scales: y = (float(sum over K of xq * wq) * xs[t]) * s[n] (a.s
 // holds one scale per row, a.ld_s = 1); y float32 or binary16 (a.y_type).
@@ -155,14 +169,14 @@ void launch_small_gemm_q8_parts(const GemmArgs& a, const SmallGemmPlan& plan, hi
 // y [t, n] (any row stride) = or += (add) the in-order sum of `parts` float32 planes part [parts][t][n].
 void launch_parts_add(int parts, bool add, std::size_t t, std::size_t n, const float* part, float* y, std::size_t ld_y,
                       hipStream_t stream);
-// One multiply of up to 64 rows (mid.hip; config -1): w8g with a 16-bit X, or q8. mid_gemm_plan returns false for what
-// the kernel does not take (another T, config or X type, offsets beyond 32 bits).
+// One w8g multiply of up to 64 rows with a 16-bit X (mid.hip; config -1). mid_gemm_plan returns false for what the kernel
+// does not take (another T, config or X type, offsets beyond 32 bits).
 struct MidGemmPlan {
     int nt;     // 16-row weight tiles per block
     int parts;  // K-parts (1 for SwiGLU)
 };
-bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan);
-void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStream_t stream);
+bool mid_gemm_plan(const GemmArgs& a, MidGemmPlan& plan);
+void launch_mid_gemm(const GemmArgs& a, const MidGemmPlan& plan, hipStream_t stream);
 // The Store / Add multiply of a float32 X of up to 24 rows (N < 8192), from its hi and lo bf16 rows (pairs: hi [t, k], then lo [t, k]).
 bool mid_pairs_plan(const GemmArgs& a, MidGemmPlan& plan);
 void launch_mid_pairs(const GemmArgs& a, const MidGemmPlan& plan, const void* pairs, hipStream_t stream);

@@ -1460,9 +1460,9 @@ void dispatch_path(const GemmArgs& a, hipStream_t stream) {
             return;
         }
     }
-    MidGemmPlan mid;  // up to 64 rows by default: K split over waves and blocks
-    if (mid_gemm_plan(a, true, mid)) {
-        launch_mid_gemm(a, true, mid, stream);
+    Q8RowsPlan rows;  // up to 64 rows by default: the kernels below, with K split over waves where their order allows
+    if (q8_rows_plan(a, rows)) {
+        launch_q8_rows(a, rows, stream);
         return;
     }
     const bool small = a.config == 1 || (a.config < 0 && q8_streams(a.t, a.n));

@@ -1459,8 +1459,8 @@ void dispatch_path(const GemmArgs& a, hipStream_t stream) {
             return;
         }
         MidGemmPlan mid;  // up to 64 rows by default: K split over waves and blocks
-        if (mid_gemm_plan(a, false, mid)) {
-            launch_mid_gemm(a, false, mid, stream);
+        if (mid_gemm_plan(a, mid)) {
+            launch_mid_gemm(a, mid, stream);
             return;
         }
     }

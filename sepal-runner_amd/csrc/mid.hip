@@ -1,5 +1,5 @@
-// The multiplies of up to 64 rows (decode batches) that the M <= 16 pass kernels do not take: Y = epilogue(X W^T) for
-// gpu-w8g (bf16 / binary16 X) and gpu-q8w.
+// The w8g multiplies of up to 64 rows (decode batches) that the M <= 16 pass kernels do not take: Y = epilogue(X W^T) for
+// bf16 / binary16 X.
 //
 // At these sizes the time to beat is one pass over the weights, as at M <= 16, but the X rows no longer fit the LDS
 // beside them (64 rows x 2560 bf16 are 320 KB), and a kernel that shares X tiles between waves spends its time on
@@ -13,14 +13,13 @@
 // The only block barriers are the two of the final sum: the waves' partial tiles meet in the slots' LDS, waves 4-7 added
 // to waves 0-3, then the four in wave order; then the epilogue. SwiGLU and one-part Store / Add write Y; a Store / Add
 // multiply too narrow to fill the chip splits K over blocks too (parts), in the workspace's partial zone, added in part
-// order by a second launch. Per group the sum of products is scaled and added in float32 (w8g: y += s_g P_g; q8: exact
-// int32 group sums, then the cpu-q8 link fma(f_g, ws_g [x xs_g], y)), so results are within float32 rounding of the
-// other paths'.
+// order by a second launch. Per group the sum of products is scaled and added in float32 (y += s_g P_g), so results are
+// within float32 rounding of the other paths'. (The q8 multiplies, whose order of links is part of their result, have
+// a kernel of their own: q8_small.hip.)
 //
 // Measured (us a call, HIP-graph replays over cold weights; before: the streaming kernel, or the large-M kernels on
-// 64-row tiles): gate/up 19456 x 2560 at 32 / 48 rows w8g 23.0 / 24.4 -> 18.7 / 21.5, q8 per token 27.8 / 38.9 -> 16.2 /
-// 17.7; down 2560 x 9728 w8g 25.4 / 24.2 -> 14.1 / 16.2, q8 per token 30.4 / 34.4 -> 12.7 / 14.3; 1024 x 4096 q8 at 48
-// rows 47 -> 7.8. What bounds it (gate/up, 48 rows, w8g, ablations): 6.5 us for an empty run of the grid, 6 for the
+// 64-row tiles): gate/up 19456 x 2560 at 32 / 48 rows 23.0 / 24.4 -> 18.7 / 21.5, down 2560 x 9728 25.4 / 24.2 -> 14.1 /
+// 16.2. What bounds it (gate/up, 48 rows, ablations): 6.5 us for an empty run of the grid, 6 for the
 // weight stream, 6.5 for the widening and the MFMAs (of which a wave overlaps little with its stream: one group of
 // NT tiles is in flight), 3 for the final sum and the epilogue; X costs 0.5.
 #include <algorithm>
@@ -33,19 +32,15 @@ namespace sepal::hip {
 namespace mid {
 
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
-// X types beyond the public ones: int8 activations (gpu-q8w) with one scale per 128 values, or per token
-constexpr int kI8 = 8, kI8Token = 9;
 
 struct Params {
-    const void* x;            // [T, ld_x] bf16 / binary16 / int8
+    const void* x;            // [T, ld_x] bf16 / binary16
     unsigned x_bytes, w_bytes, s_bytes;
     int ld_xb;                // X row stride in bytes
     const signed char* w;     // [N, ld_w]
     int ld_w;
     const float* s;           // [N, ld_s]
     int ld_s;
-    const float* xs;          // q8: activation scales [T, ld_xs], one per token or per 128 columns
-    std::size_t ld_xs;
     void* y;                  // [T, ld_y], or the parts [parts][T][N] float32
     std::size_t ld_y;
     int y_type, epilogue;     // epilogue of a one-part multiply
@@ -65,9 +60,6 @@ __device__ __forceinline__ f32x4 mfma_f(const u32x4 a, const u32x4 b, f32x4 c) {
     else
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ i32x4 mfma_i(const u32x4 a, const u32x4 b, i32x4 c) {
-    return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, a), __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
-}
 
 // s_waitcnt vmcnt(N) with the other counters left at their maximum.
 template <int N>
@@ -79,14 +71,12 @@ __device__ __forceinline__ void wait_vm() {
 // MT: 16-row tiles of X (T <= 16 MT); NT: weight tiles of a block.
 template <int XT, int MT, int NT>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) mid_kernel(const Params p) {
-    constexpr bool Q8 = XT == kI8 || XT == kI8Token, PER128 = XT == kI8;
-    constexpr int XL = Q8 ? 2 : 4;        // 16-byte X loads per lane, row tile and group
+    constexpr int XL = 4;                 // 16-byte X loads per lane, row tile and group
     constexpr int SLOT = kWaves * 2048;   // one tile's slots of all waves; the final sum's [4 waves][MT][64 lanes] x 16 B
     static_assert(4 * MT * 1024 <= SLOT, "the final sum reuses a tile's slots");
     // a separate array per tile: the compiler then knows which one a direct load writes
     __shared__ __align__(1024) unsigned char l0[SLOT], l1[NT > 1 ? SLOT : 16], l2[NT > 2 ? SLOT : 16], l3[NT > 3 ? SLOT : 16],
         l4[NT > 4 ? SLOT : 16];
-    extern __shared__ __align__(16) float xs_lds[];  // q8 per 128: [group of the part][16 MT rows]
     const auto slot = [&](auto it) -> lds_u8* {
         constexpr int i = decltype(it)::value;
         if constexpr (i == 0) return (lds_u8*)l0;
@@ -121,7 +111,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const int xrow = lane % 16, kq = lane / 16;
     int xoff[MT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) xoff[i] = min(16 * i + xrow, p.t - 1) * p.ld_xb + (Q8 ? 16 : 32) * kq;
+    for (int i = 0; i < MT; ++i) xoff[i] = min(16 * i + xrow, p.t - 1) * p.ld_xb + 32 * kq;
     // weight load e of a tile: rows 8 e + lane / 8 (SwiGLU: 8 gate rows, then the 8 up rows of the same features, 64
     // packed rows further); the lane's slot lane % 8 of its row holds chunk (lane % 8) ^ ((row / 2) % 8)
     int woff[2], wbase[NT];
@@ -150,14 +140,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const auto load_x = [&](int u, int b) __attribute__((always_inline)) {
         const bool in = u < nu;
         const __amdgpu_buffer_rsrc_t xr = rsrc(p.x, in ? p.x_bytes : 0u);
-        const int so = uniform((u0 + u) * (Q8 ? 128 : 256));
+        const int so = uniform((u0 + u) * 256);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < XL; ++j)
-                // q8: 16 bytes at 64 j + 16 kq; 16-bit X: k 64 (j / 2) + 16 kq + 8 (j % 2)
+                // k 64 (j / 2) + 16 kq + 8 (j % 2)
                 x[b][i][j] = __builtin_bit_cast(
-                    u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[i] + (Q8 ? 64 * j : 128 * (j / 2) + 16 * (j % 2)), so, 0));
+                    u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[i] + 128 * (j / 2) + 16 * (j % 2), so, 0));
     };
     const auto load_sc = [&](int u, int b) __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t sr = rsrc(p.s, u < nu ? p.s_bytes : 0u);
@@ -174,24 +164,11 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(dst + 1024), 16, woff[1], so, 0, 0);
     };
 
-    if constexpr (PER128) {
-        // the part's activation scales, requested before the weights
-        for (int id = tid; id < gpt * 16 * MT; id += kThreads) {
-            const int r = id % (16 * MT), g = id / (16 * MT);
-            xs_lds[id] = p.xs[static_cast<std::size_t>(min(r, p.t - 1)) * p.ld_xs + g_lo + g];
-        }
-    }
     load_x(0, 0);
     load_sc(0, 0);
     __builtin_amdgcn_sched_barrier(0);
     each_tile([&](auto it) { load_w(0, it); });
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (PER128) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's part of the scales is in LDS
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    }
 
     float acc[NT][MT][4];
 #pragma unroll
@@ -228,12 +205,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         constexpr int b = decltype(bt)::value;
         load_x(u + 1, b ^ 1);
         load_sc(u + 1, b ^ 1);
-        f32x4 xv[MT];
-        if constexpr (PER128) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-                xv[i] = *reinterpret_cast<const f32x4*>(xs_lds + (u0 + u - g_lo) * 16 * MT + 16 * i + 4 * kq);
-        }
         each_tile([&](auto it) __attribute__((always_inline)) {
             constexpr int t = decltype(it)::value;
             const u32x4 b0 = bw[0], b1 = bw[1];
@@ -241,42 +212,29 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
             __builtin_amdgcn_sched_barrier(0);
             wait_vm<2 * (NT - 1) + NX>();
             read(Next{});
-            if constexpr (Q8) {
+            unsigned o[16];
 #pragma unroll
-                for (int i = 0; i < MT; ++i) {
-                    i32x4 sum = mfma_i(x[b][i][0], b0, i32x4{0, 0, 0, 0});
-                    sum = mfma_i(x[b][i][1], b1, sum);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float f = PER128 ? __fmul_rn(sc[b][t], xv[i][r]) : sc[b][t];
-                        acc[t][i][r] = __builtin_fmaf(static_cast<float>(sum[r]), f, acc[t][i][r]);
-                    }
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (XT == SEPAL_HIP_BF16) {
+                    s8x4_to_bf16x4(b0[q], o[2 * q], o[2 * q + 1]);
+                    s8x4_to_bf16x4(b1[q], o[8 + 2 * q], o[9 + 2 * q]);
+                } else {
+                    s8x4_to_f16x4(b0[q], o[2 * q], o[2 * q + 1]);
+                    s8x4_to_f16x4(b1[q], o[8 + 2 * q], o[9 + 2 * q]);
                 }
-            } else {
-                unsigned o[16];
+            }
+            f32x4 prt[MT];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if constexpr (XT == SEPAL_HIP_BF16) {
-                        s8x4_to_bf16x4(b0[q], o[2 * q], o[2 * q + 1]);
-                        s8x4_to_bf16x4(b1[q], o[8 + 2 * q], o[9 + 2 * q]);
-                    } else {
-                        s8x4_to_f16x4(b0[q], o[2 * q], o[2 * q + 1]);
-                        s8x4_to_f16x4(b1[q], o[8 + 2 * q], o[9 + 2 * q]);
-                    }
-                }
-                f32x4 prt[MT];
+            for (int i = 0; i < MT; ++i) prt[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int i = 0; i < MT; ++i) prt[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int i = 0; i < MT; ++i)
-                        prt[i] = mfma_f<XT>(x[b][i][j], u32x4{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]}, prt[i]);
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
+                    prt[i] = mfma_f<XT>(x[b][i][j], u32x4{o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]}, prt[i]);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[t][i][r] = __builtin_fmaf(prt[i][r], sc[b][t], acc[t][i][r]);
-            }
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[t][i][r] = __builtin_fmaf(prt[i][r], sc[b][t], acc[t][i][r]);
             // (past the last unit the refills and the reads of empty loads are harmless)
             refill(t + 1 < NT ? u + 1 : u + 2, Next{});
         });
@@ -342,10 +300,6 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         if (i >= MT) return;
         f32x4 v = total(s, i, lane);
         const int r0 = 16 * i + 4 * (lane / 16), c = lane % 16;
-        if constexpr (Q8 && !PER128) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = __fmul_rn(v[r], p.xs[static_cast<std::size_t>(min(r0 + r, p.t - 1)) * p.ld_xs]);
-        }
         if (swiglu) {
             // gate in columns 0..7, up of the same features in columns 8..15
             const int f = 64 * (tile / 8) + 8 * (tile % 8) + c;
@@ -356,7 +310,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 if (r0 + r >= p.t) continue;
-                const float h = PER128 ? swiglu_cephes(v[r], u[r]) : swiglu_fast(v[r], u[r]);
+                const float h = swiglu_fast(v[r], u[r]);
                 const std::size_t idx = static_cast<std::size_t>(r0 + r) * p.ld_y + f;
                 if (p.y_type == SEPAL_HIP_F32) store_out<SEPAL_HIP_F32>(p.y, idx, h);
                 else if (p.y_type == SEPAL_HIP_BF16) store_out<SEPAL_HIP_BF16>(p.y, idx, h);
@@ -382,7 +336,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 // Weight tiles a block may own: five; three where 64 rows of 16-bit X fill the registers (with five tiles their next
 // group's X could only be requested behind its weights: 24.2-25.6 us at 19456 x 2560 against 23.9-24.4 of the large-M
 // kernels' plan, and 18.8 against 17.9 at 2560 x 9728).
-constexpr int max_nt(int xt, int mt) { return mt == 4 && xt != kI8 && xt != kI8Token ? 3 : 5; }
+constexpr int max_nt(int mt) { return mt == 4 ? 3 : 5; }
 
 // ---- launch ----------------------------------------------------------------------------------------------------------
 
@@ -402,52 +356,50 @@ inline int device_cus() {
 }
 
 template <int XT, int MT, int NT>
-void launch(const Params& p, std::size_t lds, hipStream_t stream) {
-    const auto kernel = mid_kernel<XT, MT, NT>;
-    if (lds > 0) raise_dynamic_lds(reinterpret_cast<const void*>(kernel), lds, "mid-M multiply");
-    kernel<<<dim3(static_cast<unsigned>(p.parts) * p.spans), dim3(kThreads), lds, stream>>>(p);
+void launch(const Params& p, hipStream_t stream) {
+    mid_kernel<XT, MT, NT><<<dim3(static_cast<unsigned>(p.parts) * p.spans), dim3(kThreads), 0, stream>>>(p);
     check_launch("mid-M multiply launch");
 }
 
 template <int XT, int MT>
-void launch_nt(const Params& p, int nt, std::size_t lds, hipStream_t stream) {
+void launch_nt(const Params& p, int nt, hipStream_t stream) {
     if (nt == 2) {
-        launch<XT, MT, 2>(p, lds, stream);
+        launch<XT, MT, 2>(p, stream);
     } else if (nt == 3) {
-        launch<XT, MT, 3>(p, lds, stream);
+        launch<XT, MT, 3>(p, stream);
     } else {
-        if constexpr (max_nt(XT, MT) >= 5) launch<XT, MT, 5>(p, lds, stream);
+        if constexpr (max_nt(MT) >= 5) launch<XT, MT, 5>(p, stream);
         else throw LaunchError("mid-M multiply: no such tile count");
     }
 }
 
 template <int XT>
-void launch_mt(const Params& p, int nt, std::size_t lds, hipStream_t stream) {
-    if (p.t <= 32) launch_nt<XT, 2>(p, nt, lds, stream);
-    else if (p.t <= 48) launch_nt<XT, 3>(p, nt, lds, stream);
-    else launch_nt<XT, 4>(p, nt, lds, stream);
+void launch_mt(const Params& p, int nt, hipStream_t stream) {
+    if (p.t <= 32) launch_nt<XT, 2>(p, nt, stream);
+    else if (p.t <= 48) launch_nt<XT, 3>(p, nt, stream);
+    else launch_nt<XT, 4>(p, nt, stream);
 }
 
 } // namespace mid
 
 namespace {
 
-bool make_plan(const GemmArgs& a, bool q8, int max_parts, MidGemmPlan& plan) {
+bool make_plan(const GemmArgs& a, int max_parts, MidGemmPlan& plan) {
     if (a.config >= 0 || a.t > kSmallM || a.w_stream || a.k % 128 != 0) return false;
-    if (!q8 && a.x_type != SEPAL_HIP_BF16 && a.x_type != SEPAL_HIP_F16) return false;
+    if (a.x_type != SEPAL_HIP_BF16 && a.x_type != SEPAL_HIP_F16) return false;
     const bool swiglu = a.epilogue == SEPAL_HIP_SWIGLU;
     if (swiglu ? a.n % 128 != 0 : (a.n % 16 != 0 || a.y_type != SEPAL_HIP_F32)) return false;
-    const std::size_t lim = std::size_t{1} << 31, xb = q8 ? 1 : 2;
-    if (a.t * a.ld_x * xb >= lim || a.n * a.ld_w >= lim || a.n * a.ld_s * 4 >= lim) return false;
+    const std::size_t lim = std::size_t{1} << 31;
+    if (a.t * a.ld_x * 2 >= lim || a.n * a.ld_w >= lim || a.n * a.ld_s * 4 >= lim) return false;
     const int cus = mid::device_cus();
     const int tiles = static_cast<int>(a.n / 16), groups = static_cast<int>(a.k / 128);
     const int mt = a.t <= 32 ? 2 : (a.t <= 48 ? 3 : 4);
-    const int max_nt = mid::max_nt(q8 ? mid::kI8 : a.x_type, mt);
+    const int max_nt = mid::max_nt(mt);
     // With three tiles a block, more than one round of blocks is slower than the large-M kernels' plan (49-64 rows of
     // 16-bit X: 32-36 against 24-25 us at 19456 x 2560, 36-41 against 25 at 20480 x 3072; level at 12288 x 2560, one
     // round).
     if (max_nt == 3 && (tiles + 2) / 3 > cus) return false;
-    const double x_kb = mt * (q8 ? 2.0 : 4.0);  // X of one group
+    const double x_kb = mt * 4.0;  // X of one group
     double best = 0.0;
     for (const int nt : {5, 3, 2}) {
         if (nt > max_nt) continue;
@@ -470,21 +422,17 @@ bool make_plan(const GemmArgs& a, bool q8, int max_parts, MidGemmPlan& plan) {
 }
 
 // The multiply alone: Y, or its K-parts [plan.parts][t][n] at part.
-void launch_multiply(const GemmArgs& a, bool q8, const MidGemmPlan& plan, float* part, hipStream_t stream) {
+void launch_multiply(const GemmArgs& a, const MidGemmPlan& plan, float* part, hipStream_t stream) {
     mid::Params p{};
-    const std::size_t xb = q8 ? 1 : 2;
     p.x = a.x;
-    p.x_bytes = static_cast<unsigned>(((a.t - 1) * a.ld_x + a.k) * xb);
-    p.ld_xb = static_cast<int>(a.ld_x * xb);
+    p.x_bytes = static_cast<unsigned>(((a.t - 1) * a.ld_x + a.k) * 2);
+    p.ld_xb = static_cast<int>(a.ld_x * 2);
     p.w = reinterpret_cast<const signed char*>(a.w);
     p.w_bytes = static_cast<unsigned>((a.n - 1) * a.ld_w + a.k);
     p.ld_w = static_cast<int>(a.ld_w);
     p.s = a.s;
     p.s_bytes = static_cast<unsigned>(((a.n - 1) * a.ld_s + a.k / 128) * 4);
     p.ld_s = static_cast<int>(a.ld_s);
-    p.xs = a.xs;
-    p.ld_xs = a.ld_xs;
-    const bool per128 = q8 && (a.act_block != a.k || a.k == 128);
     p.y = part != nullptr ? static_cast<void*>(part) : a.y;
     p.ld_y = part != nullptr ? a.n : a.ld_y;
     p.y_type = a.y_type;
@@ -495,13 +443,8 @@ void launch_multiply(const GemmArgs& a, bool q8, const MidGemmPlan& plan, float*
     p.tiles = static_cast<int>(a.n / 16);
     p.parts = plan.parts;
     p.spans = (p.tiles + plan.nt - 1) / plan.nt;
-    const int mt = p.t <= 32 ? 2 : (p.t <= 48 ? 3 : 4);
-    const std::size_t gpt = (a.k / 128 + plan.parts - 1) / plan.parts;
-    const std::size_t lds = per128 ? gpt * 16 * mt * sizeof(float) : 0;
-    if (per128) mid::launch_mt<mid::kI8>(p, plan.nt, lds, stream);
-    else if (q8) mid::launch_mt<mid::kI8Token>(p, plan.nt, lds, stream);
-    else if (a.x_type == SEPAL_HIP_BF16) mid::launch_mt<SEPAL_HIP_BF16>(p, plan.nt, lds, stream);
-    else mid::launch_mt<SEPAL_HIP_F16>(p, plan.nt, lds, stream);
+    if (a.x_type == SEPAL_HIP_BF16) mid::launch_mt<SEPAL_HIP_BF16>(p, plan.nt, stream);
+    else mid::launch_mt<SEPAL_HIP_F16>(p, plan.nt, stream);
 }
 
 float* partial_zone(const GemmArgs& a) {
@@ -521,11 +464,11 @@ GemmArgs pairs_args(const GemmArgs& a) {
 
 } // namespace
 
-bool mid_gemm_plan(const GemmArgs& a, bool q8, MidGemmPlan& plan) { return make_plan(a, q8, 16, plan); }
+bool mid_gemm_plan(const GemmArgs& a, MidGemmPlan& plan) { return make_plan(a, 16, plan); }
 
-void launch_mid_gemm(const GemmArgs& a, bool q8, const MidGemmPlan& plan, hipStream_t stream) {
+void launch_mid_gemm(const GemmArgs& a, const MidGemmPlan& plan, hipStream_t stream) {
     float* const part = plan.parts > 1 ? partial_zone(a) : nullptr;
-    launch_multiply(a, q8, plan, part, stream);
+    launch_multiply(a, plan, part, stream);
     if (part != nullptr)
         launch_parts_add(plan.parts, a.epilogue == SEPAL_HIP_ADD, a.t, a.n, part, static_cast<float*>(a.y), a.ld_y, stream);
 }
@@ -541,14 +484,14 @@ bool mid_pairs_plan(const GemmArgs& a, MidGemmPlan& plan) {
     if (a.x_type != SEPAL_HIP_F32 || a.epilogue == SEPAL_HIP_SWIGLU || a.t > 24 || a.n >= 8192) return false;
     const GemmArgs b = pairs_args(a);
     // (the sum takes 16 parts: hi and lo of up to 8)
-    return 2 * a.t * a.n * sizeof(float) <= kPartialBytes && make_plan(b, false, 8, plan);
+    return 2 * a.t * a.n * sizeof(float) <= kPartialBytes && make_plan(b, 8, plan);
 }
 
 void launch_mid_pairs(const GemmArgs& a, const MidGemmPlan& plan, const void* pairs, hipStream_t stream) {
     GemmArgs b = pairs_args(a);
     b.x = pairs;
     float* const part = partial_zone(a);
-    launch_multiply(b, false, plan, part, stream);
+    launch_multiply(b, plan, part, stream);
     // [parts][2 T][n]: each part's hi rows, then its lo rows, are two planes of [T][n]
     launch_parts_add(2 * plan.parts, a.epilogue == SEPAL_HIP_ADD, a.t, a.n, part, static_cast<float*>(a.y), a.ld_y, stream);
 }

@@ -27,7 +27,8 @@ struct StackZones {
     std::size_t end = 0;
 };
 
-StackZones stack_zones(int kind, std::size_t t, std::size_t hidden, std::size_t inter, std::size_t act_block);
+// fuse_h: q8 per 128 at 33-64 rows keeps no float32 H where the gate/up epilogue can quantize it (the same bits, slower).
+StackZones stack_zones(int kind, std::size_t t, std::size_t hidden, std::size_t inter, std::size_t act_block, bool fuse_h = false);
 
 // One call of the stack on the scratch at `ws` (laid out by stack_zones; its counter zone zero at rest). img_gate_up /
 // img_down (null, or one load-time weight image per layer): the w8g multiplies read them instead of widening the

@@ -333,9 +333,52 @@ inline int pick_gps(int spans, int groups, int mt, int xbytes, int force_splits,
     return max(1, min(gps < 1 ? 1 : gps, cap));
 }
 
+// How a problem's K is split: `splits` runs of `gps` groups (the last one shorter), each a chain of its own, added in
+// order. `lds` is the kernel's dynamic LDS.
+struct Split {
+    int spans, splits, gps;
+    std::size_t lds;
+};
+
+// Refuses (throws) what the kernel does not take.
+template <int KIND, int EP, int YT, int MT>
+Split pick_split(const GemmArgs& a) {
+    using K = Kind<KIND>;
+    Split s{};
+    s.spans = static_cast<int>((a.n + kSpan - 1) / kSpan);
+    const int groups = static_cast<int>(a.k / 128);
+    const auto kernel = gemm_stream<KIND, EP, YT, MT>;
+    const std::size_t rows = 16 * MT;
+    const auto lds_of = [&](int gps) {
+        const std::size_t x_bytes = rows * (static_cast<std::size_t>(gps) * 128 * K::xbytes + 16) +
+                                    (K::q8 ? rows * gps * sizeof(float) : 0);
+        const std::size_t tile_bytes = rows * (kSpan + 4) * sizeof(float);
+        return x_bytes > tile_bytes ? x_bytes : tile_bytes;
+    };
+    // occupancy at the largest slice this instance may take
+    const int lds_cap = ((64 << 10) / (16 * MT) - 16) / (128 * K::xbytes);  // as pick_gps
+    const int resident = resident_blocks(reinterpret_cast<const void*>(kernel), lds_of(max(1, min(kGMax, min(groups, lds_cap)))));
+    s.gps = pick_gps(s.spans, groups, MT, K::xbytes, a.force_splits, resident);
+    {
+        // no more splits than the workspace's partial zone holds (wide N at 64 rows: 5 MB per split at N = 19456)
+        const std::size_t per_split = rows * static_cast<std::size_t>(s.spans) * kSpan * sizeof(float);
+        const int max_splits = static_cast<int>(std::max<std::size_t>(1, kPartialBytes / per_split));
+        s.gps = max(s.gps, (groups + max_splits - 1) / max_splits);
+    }
+    s.splits = (groups + s.gps - 1) / s.gps;
+    require(a.force_splits != 1 || s.gps <= kGMax, "small-M multiply without a K split (config 2) takes K <= 1280");
+    s.lds = lds_of(s.gps);
+    require(s.lds <= (160u << 10) - 1024, "small-M multiply: K too long for one split (use config 1)");
+    if (s.splits > 1) {
+        const std::size_t part = static_cast<std::size_t>(s.splits) * rows * s.spans * kSpan * sizeof(float);
+        require(static_cast<std::size_t>(s.spans) * sizeof(unsigned) <= kCounterBytes && part <= kPartialBytes,
+                "small-M multiply: workspace zone too small for this shape");
+    }
+    return s;
+}
+
 template <int KIND, int EP, int YT, int MT>
 void launch_mt(const GemmArgs& a, hipStream_t stream) {
-    using K = Kind<KIND>;
     Params p{};
     p.x = a.x;
     p.ld_x = a.ld_x;
@@ -353,34 +396,13 @@ void launch_mt(const GemmArgs& a, hipStream_t stream) {
     p.t = static_cast<int>(a.t);
     p.n = static_cast<int>(a.n);
     p.k = static_cast<int>(a.k);
-    p.spans = static_cast<int>((a.n + kSpan - 1) / kSpan);
-    const int groups = p.k / 128;
     const auto kernel = gemm_stream<KIND, EP, YT, MT>;
-    const std::size_t rows = 16 * MT;
-    const auto lds_of = [&](int gps) {
-        const std::size_t x_bytes = rows * (static_cast<std::size_t>(gps) * 128 * K::xbytes + 16) +
-                                    (K::q8 ? rows * gps * sizeof(float) : 0);
-        const std::size_t tile_bytes = rows * (kSpan + 4) * sizeof(float);
-        return x_bytes > tile_bytes ? x_bytes : tile_bytes;
-    };
-    // occupancy at the largest slice this instance may take
-    const int lds_cap = ((64 << 10) / (16 * MT) - 16) / (128 * K::xbytes);  // as pick_gps
-    const int resident = resident_blocks(reinterpret_cast<const void*>(kernel), lds_of(max(1, min(kGMax, min(groups, lds_cap)))));
-    p.gps = pick_gps(p.spans, groups, MT, K::xbytes, a.force_splits, resident);
-    {
-        // no more splits than the workspace's partial zone holds (wide N at 64 rows: 5 MB per split at N = 19456)
-        const std::size_t per_split = rows * static_cast<std::size_t>(p.spans) * kSpan * sizeof(float);
-        const int max_splits = static_cast<int>(std::max<std::size_t>(1, kPartialBytes / per_split));
-        p.gps = max(p.gps, (groups + max_splits - 1) / max_splits);
-    }
-    p.splits = (groups + p.gps - 1) / p.gps;
-    require(a.force_splits != 1 || p.gps <= kGMax, "small-M multiply without a K split (config 2) takes K <= 1280");
-    const std::size_t lds = lds_of(p.gps);
-    require(lds <= (160u << 10) - 1024, "small-M multiply: K too long for one split (use config 1)");
+    const Split split = pick_split<KIND, EP, YT, MT>(a);
+    p.spans = split.spans;
+    p.splits = split.splits;
+    p.gps = split.gps;
+    const std::size_t lds = split.lds;
     if (p.splits > 1) {
-        const std::size_t part = static_cast<std::size_t>(p.splits) * rows * p.spans * kSpan * sizeof(float);
-        require(static_cast<std::size_t>(p.spans) * sizeof(unsigned) <= kCounterBytes && part <= kPartialBytes,
-                "small-M multiply: workspace zone too small for this shape");
         if (a.scratch == nullptr) throw LaunchError("small-M multiply: split-K scratch missing");
         char* ws = static_cast<char*>(a.scratch);
         p.counters = reinterpret_cast<unsigned*>(ws);
@@ -393,25 +415,26 @@ void launch_mt(const GemmArgs& a, hipStream_t stream) {
     check_launch("small-M stream kernel launch");
 }
 
-template <int KIND, int EP, int YT>
-void launch_rows(const GemmArgs& a, hipStream_t stream) {
+// f<KIND, EP, YT, MT>() for the problem's epilogue, Y type and rows.
+template <int KIND, int EP, int YT, class F>
+void for_rows(const GemmArgs& a, F&& f) {
     switch ((a.t + 15) / 16) {
-    case 1: launch_mt<KIND, EP, YT, 1>(a, stream); break;
-    case 2: launch_mt<KIND, EP, YT, 2>(a, stream); break;
-    default: launch_mt<KIND, EP, YT, 4>(a, stream); break;
+    case 1: f.template operator()<KIND, EP, YT, 1>(); break;
+    case 2: f.template operator()<KIND, EP, YT, 2>(); break;
+    default: f.template operator()<KIND, EP, YT, 4>(); break;
     }
 }
 
-template <int KIND>
-void launch_ep(const GemmArgs& a, hipStream_t stream) {
+template <int KIND, class F>
+void for_kernel(const GemmArgs& a, F&& f) {
     switch (a.epilogue) {
-    case SEPAL_HIP_STORE: launch_rows<KIND, SEPAL_HIP_STORE, SEPAL_HIP_F32>(a, stream); break;
-    case SEPAL_HIP_ADD: launch_rows<KIND, SEPAL_HIP_ADD, SEPAL_HIP_F32>(a, stream); break;
+    case SEPAL_HIP_STORE: for_rows<KIND, SEPAL_HIP_STORE, SEPAL_HIP_F32>(a, f); break;
+    case SEPAL_HIP_ADD: for_rows<KIND, SEPAL_HIP_ADD, SEPAL_HIP_F32>(a, f); break;
     default:
         switch (a.y_type) {
-        case SEPAL_HIP_F32: launch_rows<KIND, SEPAL_HIP_SWIGLU, SEPAL_HIP_F32>(a, stream); break;
-        case SEPAL_HIP_BF16: launch_rows<KIND, SEPAL_HIP_SWIGLU, SEPAL_HIP_BF16>(a, stream); break;
-        default: launch_rows<KIND, SEPAL_HIP_SWIGLU, SEPAL_HIP_F16>(a, stream); break;
+        case SEPAL_HIP_F32: for_rows<KIND, SEPAL_HIP_SWIGLU, SEPAL_HIP_F32>(a, f); break;
+        case SEPAL_HIP_BF16: for_rows<KIND, SEPAL_HIP_SWIGLU, SEPAL_HIP_BF16>(a, f); break;
+        default: for_rows<KIND, SEPAL_HIP_SWIGLU, SEPAL_HIP_F16>(a, f); break;
         }
     }
 }
@@ -419,13 +442,25 @@ void launch_ep(const GemmArgs& a, hipStream_t stream) {
 } // namespace stream
 
 void launch_stream_w8g(const GemmArgs& a, hipStream_t stream) {
-    if (a.x_type == SEPAL_HIP_BF16) stream::launch_ep<stream::KIND_W8G_BF16>(a, stream);
-    else stream::launch_ep<stream::KIND_W8G_F16>(a, stream);
+    const auto launch = [&]<int KIND, int EP, int YT, int MT>() { stream::launch_mt<KIND, EP, YT, MT>(a, stream); };
+    if (a.x_type == SEPAL_HIP_BF16) stream::for_kernel<stream::KIND_W8G_BF16>(a, launch);
+    else stream::for_kernel<stream::KIND_W8G_F16>(a, launch);
 }
 
 void launch_stream_q8(const GemmArgs& a, hipStream_t stream) {
-    if (a.act_block == a.k && a.k != 128) stream::launch_ep<stream::KIND_Q8_TOKEN>(a, stream);
-    else stream::launch_ep<stream::KIND_Q8_GROUP>(a, stream);
+    const auto launch = [&]<int KIND, int EP, int YT, int MT>() { stream::launch_mt<KIND, EP, YT, MT>(a, stream); };
+    if (a.act_block == a.k && a.k != 128) stream::for_kernel<stream::KIND_Q8_TOKEN>(a, launch);
+    else stream::for_kernel<stream::KIND_Q8_GROUP>(a, launch);
+}
+
+void stream_q8_order(const GemmArgs& a, int& splits, int& gps) {
+    const auto pick = [&]<int KIND, int EP, int YT, int MT>() {
+        const stream::Split s = stream::pick_split<KIND, EP, YT, MT>(a);
+        splits = s.splits;
+        gps = s.gps;
+    };
+    if (a.act_block == a.k && a.k != 128) stream::for_kernel<stream::KIND_Q8_TOKEN>(a, pick);
+    else stream::for_kernel<stream::KIND_Q8_GROUP>(a, pick);
 }
 
 } // namespace sepal::hip

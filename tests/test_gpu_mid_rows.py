@@ -1,6 +1,6 @@
-"""The multiplies of up to 64 rows that split K over waves and blocks (MI355X only): w8g with bf16 / binary16 X and q8 in
-both activation-scale modes, at the edges of the kernel's row tiles (16, 32, 48, 64), of its blocks of 2, 3 or 5 weight
-tiles (a last block with tiles missing), of its K-parts and of its waves (fewer groups than waves), with padded strides.
+"""The multiplies of up to 64 rows (MI355X only): w8g with bf16 / binary16 X, which splits K over waves and blocks, and q8 in
+both activation-scale modes, at the edges of the kernels' row tiles (16, 32, 48, 64), of their blocks of 2 to 8 weight
+tiles (a last block with tiles missing), of the K-parts and of the waves (fewer groups than waves), with padded strides.
 
 Reference: float64 of the dequantized operands. Bound: a float32 sum of K products and G group links is within
 (K + G + 8) 2^-24 sum |x_k w_k| of it (each product and addition rounds once; the q8 sums of a group are exact); SwiGLU
