@@ -44,6 +44,7 @@ struct Params {
     void* y;                  // [T, ld_y], or the parts [parts][T][N] float32
     std::size_t ld_y;
     int y_type, epilogue;     // epilogue of a one-part multiply
+    bool libm;                // SwiGLU by swiglu_libm
     int t, n, k;
     int tiles, parts, spans;  // 16-row weight tiles; K-parts; column spans of NT tiles
 };
@@ -301,17 +302,17 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
         f32x4 v = total(s, i, lane);
         const int r0 = 16 * i + 4 * (lane / 16), c = lane % 16;
         if (swiglu) {
-            // gate in columns 0..7, up of the same features in columns 8..15
-            const int f = 64 * (tile / 8) + 8 * (tile % 8) + c;
-            f32x4 u;
+            // gate in columns 0..7, up of the same features in columns 8..15: the lane of a gate column takes rows 0 and 1,
+            // the one of its up column rows 2 and 3
+            const bool hi = c >= 8;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) u[r] = __shfl(v[r], (lane + 8) % 64, 64);
-            if (c >= 8) return;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (r0 + r >= p.t) continue;
-                const float h = swiglu_fast(v[r], u[r]);
-                const std::size_t idx = static_cast<std::size_t>(r0 + r) * p.ld_y + f;
+            for (int j = 0; j < 2; ++j) {
+                const float own = hi ? v[j + 2] : v[j], other = __shfl_xor(hi ? v[j] : v[j + 2], 8, 64);
+                const float gate = hi ? other : own, up = hi ? own : other;
+                const int row = r0 + j + (hi ? 2 : 0);
+                const float h = p.libm ? swiglu_libm(gate, up) : swiglu_fast(gate, up);
+                if (row >= p.t) continue;
+                const std::size_t idx = static_cast<std::size_t>(row) * p.ld_y + 64 * (tile / 8) + 8 * (tile % 8) + c % 8;
                 if (p.y_type == SEPAL_HIP_F32) store_out<SEPAL_HIP_F32>(p.y, idx, h);
                 else if (p.y_type == SEPAL_HIP_BF16) store_out<SEPAL_HIP_BF16>(p.y, idx, h);
                 else store_out<SEPAL_HIP_F16>(p.y, idx, h);
@@ -437,6 +438,12 @@ void launch_multiply(const GemmArgs& a, const MidGemmPlan& plan, float* part, hi
     p.ld_y = part != nullptr ? a.n : a.ld_y;
     p.y_type = a.y_type;
     p.epilogue = a.epilogue;
+    // the silu of the kernels that ran, and run what this one refuses, at these sizes: the streaming kernel's up to 32 rows with
+    // N < 8192 (closer to silu(g) u by a third in rms, and finite where g u is not), the large-M kernels' elsewhere
+    // (the libm form there, on the gate columns' lanes alone, took 19.9 / 25.0 us at 19456 x 2560 and 17 / 48 rows against
+    // 17.4 / 21.8; with the lanes shared as now 4096 x 1024 at 17 / 32 rows takes 6.7 / 7.6 with it and 6.3 / 7.1 took the
+    // fast form before)
+    p.libm = a.t <= 32 && a.n < 8192;
     p.t = static_cast<int>(a.t);
     p.n = static_cast<int>(a.n);
     p.k = static_cast<int>(a.k);

@@ -129,3 +129,27 @@ def test_float32_x(sm, t, n, k):
     sm.gemm_w8g(x, q, s, y=y[:, :n], epilogue=sm.ADD)
     _check(y[:, :n], 2 * ref, 2 * mag, u)
     assert torch.equal(sm.gemm_w8g(x, q, s), first)
+
+
+@pytest.mark.parametrize("t,n", [(1, 128), (17, 128), (18, 384), (32, 4096), (32, 8064)])
+def test_swiglu_of_exact_sums(sm, t, n):
+    """One product a sum and weight scales of powers of two: gate and up are exact, so the default SwiGLU up to 32 rows with
+    N < 8192 differs from the weight-streaming path's (config 1) only in its silu, which is the same function: equal
+    bits, also where gate times up leaves float32 beside a vanishing silu."""
+    print("[case] mid swiglu", t, n, flush=True)
+    k = 128
+    g = torch.Generator(device="cuda").manual_seed(t + n)
+    w = torch.zeros(n, k, dtype=torch.int8, device="cuda")
+    gate = (torch.arange(n, device="cuda") // 64) % 2 == 0
+    w[gate, 0], w[~gate, 1] = 1, 1
+    s = torch.exp2(torch.randint(-3, 3, (n, 1), generator=g, device="cuda").float())
+    x = torch.zeros(t, k, device="cuda")
+    x[:, 0] = torch.randn(t, generator=g, device="cuda") * 8
+    x[:, 1] = torch.randn(t, generator=g, device="cuda")
+    x[0, 0], x[0, 1] = -1e4, 3e37
+    if t > 1:
+        x[1, 0], x[1, 1] = -90.0, 1e37
+    for dt in (torch.bfloat16, torch.float16, torch.float32):
+        y = sm.gemm_w8g(x.bfloat16(), w, s, epilogue=sm.SWIGLU, y_dtype=dt)
+        assert not torch.isnan(y).any()
+        assert torch.equal(y, sm.gemm_w8g(x.bfloat16(), w, s, epilogue=sm.SWIGLU, y_dtype=dt, config=1))
