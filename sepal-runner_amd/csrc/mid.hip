@@ -27,6 +27,7 @@
 
 #include "common.hpp"
 #include "gemm_kernels.hpp"
+#include "group_window.hpp"
 
 namespace sepal::hip {
 namespace mid {
@@ -108,7 +109,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     const int u0 = g_lo + wave * base + min(wave, rem);
 
     // ---- addresses: 32-bit lane offsets, the group and the tile in the scalar offset; a group past the wave's range is
-    // loaded through a descriptor of no bytes (zeros, no memory access), so every step issues the same loads ----
+    // loaded through an empty window (group_window), so every step issues the same loads ----
     const int xrow = lane % 16, kq = lane / 16;
     int xoff[MT];
 #pragma unroll
@@ -139,9 +140,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     float sc[2][NT];
     // X and the weight scales of unit u into set b
     const auto load_x = [&](int u, int b) __attribute__((always_inline)) {
-        const bool in = u < nu;
-        const __amdgpu_buffer_rsrc_t xr = rsrc(p.x, in ? p.x_bytes : 0u);
-        const int so = uniform((u0 + u) * 256);
+        const Window win = group_window(u < nu, p.x_bytes, (u0 + u) * 256);
+        const __amdgpu_buffer_rsrc_t xr = rsrc(p.x, win.bytes);
+        const int so = uniform(win.scalar);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -151,16 +152,19 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                     u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, xoff[i] + 128 * (j / 2) + 16 * (j % 2), so, 0));
     };
     const auto load_sc = [&](int u, int b) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t sr = rsrc(p.s, u < nu ? p.s_bytes : 0u);
+        const Window win = group_window(u < nu, p.s_bytes, (u0 + u) * 4);
+        const __amdgpu_buffer_rsrc_t sr = rsrc(p.s, win.bytes);
+        const int so = uniform(win.scalar);
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-            sc[b][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, soff[t], uniform((u0 + u) * 4), 0));
+            sc[b][t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, soff[t], so, 0));
     };
     const auto load_w = [&](int u, auto it) __attribute__((always_inline)) {
         constexpr int t = decltype(it)::value;
-        const __amdgpu_buffer_rsrc_t wr = rsrc(p.w, u < nu ? p.w_bytes : 0u);
+        const Window win = group_window(u < nu, p.w_bytes, wbase[t] + 128 * (u0 + u));
+        const __amdgpu_buffer_rsrc_t wr = rsrc(p.w, win.bytes);
         lds_u8* dst = slot(it) + wave * 2048;
-        const int so = uniform(wbase[t] + 128 * (u0 + u));
+        const int so = uniform(win.scalar);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)dst, 16, woff[0], so, 0, 0);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(dst + 1024), 16, woff[1], so, 0, 0);
     };

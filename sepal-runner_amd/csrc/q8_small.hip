@@ -22,6 +22,7 @@
 
 #include "common.hpp"
 #include "gemm_kernels.hpp"
+#include "group_window.hpp"
 
 namespace sepal::hip {
 namespace q8s {
@@ -103,9 +104,8 @@ __global__ void __launch_bounds__(64 * WT) rows_kernel(const Params p) {
     const int tile = min(my_tile, p.tiles - 1);  // tiles past the last repeat it and are never stored
     const bool swiglu = p.epilogue == SEPAL_HIP_SWIGLU;
 
-    // 32-bit lane offsets, the group in the scalar offset; a group past the run is loaded through a descriptor of no bytes
-    // (zeros and no memory access: the range check covers the scalar offset, without wrapping), so that every step issues
-    // the same loads
+    // 32-bit lane offsets, the group in the scalar offset; a group past the run is loaded through an empty window
+    // (group_window), so that every step issues the same loads
     const int c = lane % 16, kq = lane / 16;
     // X load e fills kilobyte e of a stage = rows 8 e + {0..7}; lane l writes slot l % 8 of row 8 e + l / 8, which holds
     // chunk (l % 8) ^ ((row / 2) % 8); rows past T repeat the last
@@ -131,13 +131,14 @@ __global__ void __launch_bounds__(64 * WT) rows_kernel(const Params p) {
     const auto issue = [&](int u, auto it) __attribute__((always_inline)) {
         constexpr int b = decltype(it)::value % D;
         const bool in = u < nu;
-        const __amdgpu_buffer_rsrc_t xr = rsrc(p.x, in ? p.x_bytes : 0u), wr = rsrc(p.w, in ? p.w_bytes : 0u),
-                                     sr = rsrc(p.ws, in ? p.ws_bytes : 0u);
-        const int so = uniform((g_lo + u) * 128);
+        const Window xw = group_window(in, p.x_bytes, (g_lo + u) * 128), ww = group_window(in, p.w_bytes, (g_lo + u) * 128),
+                     sw = group_window(in, p.ws_bytes, (g_lo + u) * 4);
+        const __amdgpu_buffer_rsrc_t xr = rsrc(p.x, xw.bytes), wr = rsrc(p.w, ww.bytes), sr = rsrc(p.ws, sw.bytes);
+        const int so = uniform(xw.scalar), s_so = uniform(sw.scalar);  // (X and W rows advance alike)
         lds_u8* const dst = stage(it);
 #pragma unroll
         for (int q = 0; q < XW; ++q) load_kb(xr, dst + xe[q] * 1024, xoff[q], so);
-        sc[b] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, soff, uniform((g_lo + u) * 4), 0));
+        sc[b] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, soff, s_so, 0));
 #pragma unroll
         for (int j = 0; j < 2; ++j)
             wb[b][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, woff + 64 * j, so, 0));
