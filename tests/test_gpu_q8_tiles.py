@@ -28,10 +28,13 @@ def host(t):
     return t.cpu().numpy()
 
 
-# t, n, k (256 CUs): 32 x 128; 64 x 128; 96 x 128; 128 x 128; 128 x 256; one and two rounds of 128 x 256 and the rest small;
-# a round of 128 x 256 and parts of the rest's tiles wholly past T
+# t, n, k: 32 x 128; 64 x 128; 96 x 128; 128 x 128; 128 x 256; one and two rounds of 128 x 256 and the rest small; a round of
+# 128 x 256 and parts of the rest's tiles wholly past T; small tiles of which a block takes several in turn, the scale ring
+# carried on from one to the next (test_launch_rules.py holds the plan to these)
 SHAPES = [(65, 2560, 384), (300, 2576, 384), (450, 2560, 768), (897, 2560, 768), (1300, 2576, 768), (2100, 2560, 384),
-          (511, 19456, 2560), (900, 19456, 2560), (97, 128, 128), (66, 16, 256), (3872, 2560, 1280), (2200, 4352, 1280)]
+          (511, 19456, 2560), (900, 19456, 2560), (97, 128, 128), (66, 16, 256), (3872, 2560, 1280), (2200, 4352, 1280),
+          (129, 21776, 128), (257, 22272, 640), (920, 8368, 1152), (1988, 4224, 1024), (546, 16176, 1536), (8235, 784, 512),
+          (1439, 7024, 4352)]
 
 
 @pytest.mark.parametrize("act", ["token", "128"])
@@ -73,3 +76,22 @@ def test_chain_tiles(sm, t, n, k, act):
             hq, hs = sm.gemm_q8_swiglu_quantize(xq, xs, wq, ws, act_block=block)
             rq, rs = sm.quantize_rows_s8(h, block=128)
             assert torch.equal(hq, rq) and torch.equal(hs, rs)
+
+
+@pytest.mark.parametrize("act", ["token", "128"])
+def test_row_stride_past_32_bit_offsets(sm, act):
+    """Y rows 2^20 values apart: an edge tile's stores go by 64-bit addresses; the contiguous call's values, and nothing
+    between the rows written."""
+    t, n, k, ld = 70, 272, 384, 1 << 20
+    print("[case] q8 row stride", t, n, k, ld, act, flush=True)
+    block = k if act == "token" else 128
+    g = torch.Generator(device="cuda").manual_seed(t)
+    wq, ws = sm.quantize_group_s8(torch.randn(n, k, generator=g, device="cuda") * 0.02, rule=1)
+    xq, xs = sm.quantize_rows_s8(torch.randn(t, k, generator=g, device="cuda"), block=block)
+    y = torch.full((t, ld), 7.0, device="cuda")
+    for epilogue, cols, weights, scales in ((sm.STORE, n, wq, ws), (sm.ADD, n, wq, ws), (sm.SWIGLU, 128, wq[:256], ws[:256])):
+        y.fill_(7.0)
+        want = torch.full((t, cols), 7.0, device="cuda")
+        sm.gemm_q8(xq, xs, weights, scales, y=want, epilogue=epilogue, act_block=block)
+        sm.gemm_q8(xq, xs, weights, scales, y=y[:, :cols], epilogue=epilogue, act_block=block)
+        assert torch.equal(y[:, :cols], want) and (y[:, cols:] == 7.0).all()

@@ -42,3 +42,62 @@ int main() {
 }
 """)
     assert out.split() == ["0", "0"]
+
+
+CHAIN, INT8_OUT, WHOLE = 0, 1, 2  # as chain_plan's kinds
+TOKEN, PER128 = 0, 1
+
+# (t, n, k), kind, activation scales -> whole 128 x 256 tiles first, the tile of the rest, whether a block takes several:
+# the shapes of test_gpu_q8_tiles.py and test_gpu_s8_tiles.py, which mean to run these
+PLANS = [
+    ((65, 2560, 384), CHAIN, PER128, (0, "32x128", False)),
+    ((450, 2560, 768), CHAIN, TOKEN, (0, "64x128", False)),
+    ((897, 2560, 768), CHAIN, PER128, (0, "96x128", False)),
+    ((1300, 2576, 768), CHAIN, TOKEN, (0, "128x128", False)),
+    ((2100, 2560, 384), CHAIN, PER128, (0, "128x256", False)),
+    ((511, 19456, 2560), CHAIN, TOKEN, (256, "64x128", False)),
+    ((511, 19456, 2560), INT8_OUT, PER128, (256, "64x256", False)),
+    ((900, 19456, 2560), CHAIN, PER128, (512, "128x128", False)),
+    ((129, 21776, 128), CHAIN, PER128, (0, "32x128", True)),
+    ((257, 22272, 640), CHAIN, TOKEN, (0, "64x128", True)),
+    ((257, 22272, 640), CHAIN, PER128, (0, "64x128", True)),
+    ((257, 22272, 640), INT8_OUT, PER128, (0, "64x256", True)),
+    ((920, 8368, 1152), CHAIN, PER128, (0, "64x128", True)),
+    ((1988, 4224, 1024), CHAIN, PER128, (0, "96x128", True)),
+    ((546, 16176, 1536), CHAIN, TOKEN, (0, "96x128", True)),
+    ((8235, 784, 512), CHAIN, TOKEN, (0, "128x128", True)),
+    ((1439, 7024, 4352), CHAIN, PER128, (0, "128x128", True)),
+    ((65, 2560, 400), WHOLE, TOKEN, (0, "64x128", False)),
+    ((65, 2560, 2576), WHOLE, TOKEN, (0, "32x128", False)),
+    ((90, 2574, 1296), WHOLE, TOKEN, (0, "32x128", False)),
+    ((1024, 2560, 1136), WHOLE, TOKEN, (0, "96x128", False)),
+    ((1500, 2560, 528), WHOLE, TOKEN, (0, "128x128", False)),
+    ((2100, 2560, 256), WHOLE, TOKEN, (0, "128x256", False)),
+    ((3872, 2560, 2560), WHOLE, TOKEN, (256, "64x128", False)),
+    ((257, 21808, 400), WHOLE, TOKEN, (0, "64x128", True)),
+    ((6494, 1330, 1792), WHOLE, TOKEN, (0, "96x128", True)),
+    ((8221, 784, 272), WHOLE, TOKEN, (0, "128x128", True)),
+]
+
+
+def test_chain_plan(tmp_path):
+    """The tiles that the tests' shapes are there for, on 256 CUs."""
+    numbers = [v for shape, kind, act, _ in PLANS for v in (*shape, kind, act)]
+    out = _run(tmp_path, r"""
+#include <cstdio>
+#include <cstdlib>
+#include "chain_plan.hpp"
+using namespace sepal::hip::q8;
+int main(int argc, char** argv) {
+    const int cus = 256;
+    for (int i = 1; i + 4 < argc; i += 5) {
+        const int t = std::atoi(argv[i]), n = std::atoi(argv[i + 1]), k = std::atoi(argv[i + 2]);
+        const ChainPlan p = chain_plan(t, n, k / 128, std::atoi(argv[i + 3]), std::atoi(argv[i + 4]) != 0, cus);
+        const int rows = p.tile->rows(), cols = p.tile->cols(), big = (t + 127) / 128 * ((n + 255) / 256);
+        const int tiles = p.full > 0 ? (big - p.full) * (128 / rows) * (256 / cols) : (t + rows - 1) / rows * ((n + cols - 1) / cols);
+        std::printf("%d %dx%d %d\n", p.full, rows, cols, tiles > p.tile->per_cu * cus);
+    }
+}
+""", *numbers)
+    got = [(int(a), b, c == "1") for a, b, c in (line.split() for line in out.splitlines())]
+    assert got == [want for *_, want in PLANS]
