@@ -87,11 +87,14 @@ SEPAL_HIP_API int32_t sepal_hip_quantize_gate_up_s8(const void* gate, const void
  * 16 bytes). Pointers: W and Y 16-byte aligned, a float32 X too (a 16-bit X may have any alignment). The kernels read
  * 16-bit X rows of whole 16-byte chunks and store STORE / ADD outputs in 16-column tiles; other strides and the last
  * N mod 16 columns are staged in the workspace (a contiguous copy of X; one zero-padded 16-row weight tile whose
- * float32 outputs are stored or added into Y). `config` -1 picks a path by T and N (at
- * T <= 16 with a 16-bit X the M <= 16 stack's pass kernels where the shape fits them; at T <= 64 with a 16-bit X a
- * kernel that splits K over waves and blocks, at 49 to 64 rows for N <= 48 x CUs only; on the large-M path grids too small to fill the chip may split K over blocks; a row's bits then depend on
- * T); 0 forces the large-M
- * tiled path without a split of K (a row's bits do not depend on the batch, as the reference's), 1 the small-M
+ * float32 outputs are stored or added into Y). `config` -1 picks a path by T and N. With a 16-bit X:
+ * at T <= 16 the M <= 16 stack's pass kernels where the shape fits them; at T <= 64 a kernel that splits K over waves and
+ * blocks, at 49 to 64 rows for N <= 48 x CUs only; small-M streaming for what these do not take (offsets beyond 32 bits)
+ * at T <= 32 with N < 8192; the large-M tiled path otherwise, where grids too small to fill the chip may split K over
+ * blocks. With a float32 X: at T <= 24 with N < 8192 (STORE / ADD) its hi and lo rows as one multiply of the K-splitting
+ * kernel; at T <= 32 with N < 8192 otherwise the hi and the lo rows as two multiplies of a 16-bit X, added in float32;
+ * else the large-M path over the hi + lo row. Each of these rounds in its own order, so a row's bits depend on T. 0 forces
+ * the large-M tiled path without a split of K (a row's bits do not depend on the batch, as the reference's), 1 the small-M
  * weight-streaming path, 2 the small-M path without a split of K (the whole K of a column block in one block; K at
  * most 1280).
  * Replaces launch_gemm_simt with SimtWeight::Int8Group (runner/cuda/src/gemm_simt_kernels.hpp:55-57, .cu:312-332). */
