@@ -1224,7 +1224,9 @@ struct SmallGridPlan {
 // every plan): the time per 128-value group of a lone block of 64, 128 or 256 rows (MB 1, 2, 4); the rate at which
 // the blocks' operand reads are served; the in-kernel split hand-off, a fixed cost plus the last block's reads of the
 // S partials of its tile (one block's coherent reads are slow); or the planes' finisher, a launch plus the S planes
-// read and the output written at the rate of a plain streaming kernel. Negative: the plan does not fit the scratch.
+// read and the output written at the rate of a plain streaming kernel. The times are a 16-bit X's: the hi + lo form of a
+// float32 X takes about twice the compute per group, so for it the model undervalues splits. Negative: the plan does not
+// fit the scratch.
 inline double grid_cost(long t, int tiles_n, int groups, int mb, int sp, bool planes, int cus) {
     constexpr double us_per_group[5] = {0.0, 1.65, 2.44, 0.0, 4.60};
     constexpr double operand_bytes_per_us = 9.27e6, handoff_us = 5.7, tail_bytes_per_us = 8.8e4;

@@ -10,8 +10,9 @@
 //            group as soon as its operands are in registers, so a wave keeps NT - 1 to NT slots in flight (80 KB a CU);
 //   X        straight into registers in MFMA operand order (every wave has its own groups, so no X value is read twice
 //            by a block; the blocks' re-reads are L2 hits), one group ahead.
-// The only block barriers are the two of the final sum: the waves' partial tiles meet in the slots' LDS, waves 4-7 added
-// to waves 0-3, then the four in wave order; then the epilogue. SwiGLU and one-part Store / Add write Y; a Store / Add
+// The only block barriers are the three of the final sum (the slots are free, waves 4-7 have written, their sums with waves
+// 0-3 are written): the waves' partial tiles meet in the slots' LDS, waves 4-7 added to waves 0-3, then the four in wave
+// order; then the epilogue. SwiGLU and one-part Store / Add write Y; a Store / Add
 // multiply too narrow to fill the chip splits K over blocks too (parts), in the workspace's partial zone, added in part
 // order by a second launch. Per group the sum of products is scaled and added in float32 (y += s_g P_g), so results are
 // within float32 rounding of the other paths'. (The q8 multiplies, whose order of links is part of their result, have
