@@ -125,7 +125,7 @@ SEPAL_HIP_API int32_t sepal_hip_quantize_rows_s8(const void* x, int32_t x_type, 
  * [T, ld_y], or y_type for SWIGLU. K a multiple of 128; strides multiples of 16; 16-byte aligned pointers. `config`
  * -1 has the bits of the small-M path up to 64 rows (above 32 rows only for N < 8192; at T <= 16 with a float32 Y the
  * M <= 16 stack's q8 passes run where the shape fits them, with an order of their own) and of the large-M path
- * otherwise; 0 forces the large-M path, 1 the streaming small-M path, 2 the streaming path with the chain whole; the
+ * otherwise, also for what the small-M path refuses (config 1: a run too long for the LDS); 0 forces the large-M path, 1 the streaming small-M path, 2 the streaming path with the chain whole; the
  * small-M path splits K into runs, which keeps the int32 group sums exact but adds the runs' partial chains in order
  * (within tolerance, not bit for bit); config 2 keeps the chain whole (bit for bit).
  * Replaces kernel_i8_z + finish_tile (runner/src/cpu/gemm_kernels_avx512.cpp:67-115, gemm.cpp:417-447, 545-569)

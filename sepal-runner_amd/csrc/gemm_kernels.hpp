@@ -9,7 +9,8 @@ namespace sepal::hip {
 inline constexpr std::size_t kSmallM = 64;
 
 // Whose order of links the q8 multiply keeps by default (config -1) up to kSmallM rows: true, the small-M (streaming)
-// kernels' (runs of groups, stream_q8_order); false, the whole chain of the large-M kernels, cpu-q8 bit for bit. The
+// kernels' (runs of groups, stream_q8_order; the whole chain where those refuse the shape: an N whose runs' sums exceed the
+// partial zone unless a run is too long for the LDS); false, the whole chain of the large-M kernels, cpu-q8 bit for bit. The
 // kernels themselves run what launch_q8_rows refuses.
 inline bool q8_streams(std::size_t t, std::size_t n) { return t <= kSmallM && (t <= 32 || n < 8192); }
 
@@ -80,8 +81,8 @@ inline std::size_t gemm_w8g_split_bytes(const GemmArgs& a) { return (a.t * a.k *
 void launch_stream_w8g(const GemmArgs& a, hipStream_t stream);
 void launch_stream_q8(const GemmArgs& a, hipStream_t stream);
 // The order of links of launch_stream_q8: `splits` runs of `gps` groups (the last shorter), each a chain from +0, added in
-// order. Refuses (throws) what that kernel does not take.
-void stream_q8_order(const GemmArgs& a, int& splits, int& gps);
+// order. False for what that kernel does not take.
+bool stream_q8_order(const GemmArgs& a, int& splits, int& gps);
 // One q8 multiply of up to 64 rows (q8_small.hip; config -1), with the bits of the kernel that q8_streams names.
 // q8_rows_plan returns false for what the kernel does not take (another T or config, offsets beyond 32 bits, a run's scales
 // beyond the LDS).

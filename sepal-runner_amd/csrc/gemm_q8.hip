@@ -1390,12 +1390,13 @@ void dispatch_path(const GemmArgs& a, hipStream_t stream) {
             return;
         }
     }
-    Q8RowsPlan rows;  // up to 64 rows by default: the kernels below, with K split over waves where their order allows
+    Q8RowsPlan rows;  // up to 64 rows by default, the bits of the kernels below
     if (q8_rows_plan(a, rows)) {
         launch_q8_rows(a, rows, stream);
         return;
     }
-    const bool small = a.config == 1 || (a.config < 0 && q8_streams(a.t, a.n));
+    int splits, gps;
+    const bool small = a.config == 1 || (a.config < 0 && q8_streams(a.t, a.n) && stream_q8_order(a, splits, gps));
     if (small) launch_stream_q8(a, stream);
     else launch_big<EP, YT, PT, MODE_CHAIN>(a, stream);
 }

@@ -408,10 +408,11 @@ bool q8_rows_plan(const GemmArgs& a, Q8RowsPlan& plan) {
     if (swiglu ? a.n % 128 != 0 : (a.n % 16 != 0 || a.y_type != SEPAL_HIP_F32)) return false;
     const std::size_t lim = std::size_t{1} << 31;
     if (a.t * a.ld_x >= lim || a.n * a.ld_w >= lim || a.n * a.ld_s * 4 >= lim) return false;
-    plan.whole = !q8_streams(a.t, a.n);
-    plan.splits = 1;
-    plan.gps = static_cast<int>(a.k / 128);
-    if (!plan.whole) stream_q8_order(a, plan.splits, plan.gps);
+    plan.whole = !q8_streams(a.t, a.n) || !stream_q8_order(a, plan.splits, plan.gps);
+    if (plan.whole) {
+        plan.splits = 1;
+        plan.gps = static_cast<int>(a.k / 128);
+    }
     const bool per128 = a.act_block != a.k || a.k == 128;
     return q8_rows_blocks(a.t <= 32 ? 2 : (a.t <= 48 ? 3 : 4), per128, static_cast<int>(a.n / 16), static_cast<int>(a.k / 128), plan.splits, plan.gps,
                           q8s::device_cus(), plan);

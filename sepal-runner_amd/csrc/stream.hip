@@ -338,9 +338,9 @@ inline int pick_gps(int spans, int groups, int mt, int xbytes, int force_splits,
 struct Split {
     int spans, splits, gps;
     std::size_t lds;
+    const char* refused;  // why the kernel does not take the problem, or null
 };
 
-// Refuses (throws) what the kernel does not take.
 template <int KIND, int EP, int YT, int MT>
 Split pick_split(const GemmArgs& a) {
     using K = Kind<KIND>;
@@ -366,14 +366,12 @@ Split pick_split(const GemmArgs& a) {
         s.gps = max(s.gps, (groups + max_splits - 1) / max_splits);
     }
     s.splits = (groups + s.gps - 1) / s.gps;
-    require(a.force_splits != 1 || s.gps <= kGMax, "small-M multiply without a K split (config 2) takes K <= 1280");
     s.lds = lds_of(s.gps);
-    require(s.lds <= (160u << 10) - 1024, "small-M multiply: K too long for one split (use config 1)");
-    if (s.splits > 1) {
-        const std::size_t part = static_cast<std::size_t>(s.splits) * rows * s.spans * kSpan * sizeof(float);
-        require(static_cast<std::size_t>(s.spans) * sizeof(unsigned) <= kCounterBytes && part <= kPartialBytes,
-                "small-M multiply: workspace zone too small for this shape");
-    }
+    const std::size_t part = static_cast<std::size_t>(s.splits) * rows * s.spans * kSpan * sizeof(float);
+    if (a.force_splits == 1 && s.gps > kGMax) s.refused = "small-M multiply without a K split (config 2) takes K <= 1280";
+    else if (s.lds > (160u << 10) - 1024) s.refused = "small-M multiply: K too long for one split (use config 1)";
+    else if (s.splits > 1 && (static_cast<std::size_t>(s.spans) * sizeof(unsigned) > kCounterBytes || part > kPartialBytes))
+        s.refused = "small-M multiply: workspace zone too small for this shape";
     return s;
 }
 
@@ -398,6 +396,7 @@ void launch_mt(const GemmArgs& a, hipStream_t stream) {
     p.k = static_cast<int>(a.k);
     const auto kernel = gemm_stream<KIND, EP, YT, MT>;
     const Split split = pick_split<KIND, EP, YT, MT>(a);
+    require(split.refused == nullptr, split.refused != nullptr ? split.refused : "");
     p.spans = split.spans;
     p.splits = split.splits;
     p.gps = split.gps;
@@ -453,14 +452,17 @@ void launch_stream_q8(const GemmArgs& a, hipStream_t stream) {
     else stream::for_kernel<stream::KIND_Q8_GROUP>(a, launch);
 }
 
-void stream_q8_order(const GemmArgs& a, int& splits, int& gps) {
+bool stream_q8_order(const GemmArgs& a, int& splits, int& gps) {
+    bool taken = false;
     const auto pick = [&]<int KIND, int EP, int YT, int MT>() {
         const stream::Split s = stream::pick_split<KIND, EP, YT, MT>(a);
+        taken = s.refused == nullptr;
         splits = s.splits;
         gps = s.gps;
     };
     if (a.act_block == a.k && a.k != 128) stream::for_kernel<stream::KIND_Q8_TOKEN>(a, pick);
     else stream::for_kernel<stream::KIND_Q8_GROUP>(a, pick);
+    return taken;
 }
 
 } // namespace sepal::hip

@@ -69,6 +69,24 @@ def test_default_bits(sm, t, n, k, act):
         assert torch.equal(qa, qb) and torch.equal(_bits(sa), _bits(sb))
 
 
+# t, n, k: runs' sums beyond the workspace's zone unless a run is too long for the streaming kernel's LDS; per 128 the scales
+# of the whole chain beyond a block's LDS array (the large-M kernels), and within it
+@pytest.mark.parametrize("act", ["token", "128"])
+@pytest.mark.parametrize("t,n,k", [(64, 8176, 40960), (32, 135168, 4992)])
+def test_shapes_the_streaming_kernel_refuses(sm, t, n, k, act):
+    """The default has the whole chain there (config 0); config 1 stays refused."""
+    print("[case] q8 order, refused by the streaming kernel", t, n, k, act, flush=True)
+    block = k if act == "token" else 128
+    xq, xs, w, ws = _operands(sm, t, n, k, block)
+    with pytest.raises(sm.SepalHipInvalid):
+        sm.gemm_q8(xq, xs, w, ws, act_block=block, config=1)
+    for epilogue in (sm.STORE, sm.ADD):
+        a, b = torch.ones(t, n, device="cuda"), torch.ones(t, n, device="cuda")
+        sm.gemm_q8(xq, xs, w, ws, y=a, epilogue=epilogue, act_block=block)
+        sm.gemm_q8(xq, xs, w, ws, y=b, epilogue=epilogue, act_block=block, config=0)
+        assert torch.equal(_bits(a), _bits(b))
+
+
 def test_whole_chain_is_cpu_q8(sm):
     t, n, k = 33, 8192, 1408
     xq, xs, w, ws = _operands(sm, t, n, k, 128)
